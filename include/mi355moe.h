@@ -321,6 +321,7 @@ int mi_dequant(const mi_table *t, int32_t expert, float *out, void *stream);
 #define MI_I8_COL_SCALES 1
 #define MI_I8_COL_AFTER  2
 #define MI_I8_TILED      0x100
+#define MI_W_BF16        3       /* mi_mlp_many only: bf16 weights, no scales */
 int mi_int8_project(const uint16_t *x_bf16, int32_t B, const int8_t *qT, const float *s, int32_t scale_axis,
                     int32_t n_in, int32_t n_out, uint16_t *y_bf16, float *y_f32, void *workspace,
                     size_t workspace_bytes, void *stream);
@@ -390,12 +391,26 @@ int mi_bf16_mlp(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I, const u
 size_t mi_bf16_mlp_workspace(int32_t B, int32_t D, int32_t I);
 
 /*
+ * mlp_partial for many tokens (a prompt piece; 1 <= B <= 16384): the steps, shapes, weight layouts and rounding points
+ * of mi_int8_mlp and mi_bf16_mlp, as dense GEMMs that meet a weight tile with up to 128 tokens.  gu_form / down_form:
+ * MI_I8_ROW_SCALES or MI_I8_COL_SCALES (| MI_I8_TILED) over int8, or MI_W_BF16.  x, the weights, y_f32, the workspace
+ * and per-row scales 16-byte aligned, y_bf16 8-byte.  Workspace: mi_mlp_many_workspace bytes, no counters: its
+ * contents need no initialisation.
+ */
+int mi_mlp_many(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I, const void *gate_w, const float *gate_s,
+                const void *up_w, const float *up_s, int32_t gu_form, const void *down_w, const float *down_s,
+                int32_t down_form, float limit, uint16_t *y_bf16, float *y_f32, void *workspace,
+                size_t workspace_bytes, void *stream);
+size_t mi_mlp_many_workspace(int32_t B, int32_t D, int32_t I);
+
+/*
  * Launch-plan overrides, for tests and measurement runs only (no counterpart in the reference).  The library reads
  * no environment variables: every call plans its launches from built-in defaults, except for the names set here,
  * which replace those defaults process-wide until mi_tuning_reset.  Names (an unknown one gives MI_ERR_ARG):
  * split counts and row tiles of the decode launch families (S1, S2, FS1, FS2, SMV, each with _RTW and _AL; MS1, MS2,
  * CS1, CS2 with _RTW; MGMAX), launch-family switches (CUSTREAM, CUMULTI, PERSIST_ABOVE, FUSE_SWIGLU, CU_FORM_H), the
- * one-launch decode's poll limit (SPIN_LIMIT) and the int8 split plan (I8S, I8_WAVES, I8_FUSE).  Overrides change
+ * one-launch decode's poll limit (SPIN_LIMIT), the int8 split plan (I8S, I8_WAVES, I8_FUSE) and the many-token MLP's
+ * splits and token tile (DG_S1, DG_S2, DG_NT).  Overrides change
  * launch shapes and summation orders, never the result beyond f32 rounding; workspace sizes follow them, so set them
  * before sizing a workspace.  Not synchronised with calls running on other host threads.
  */

@@ -21,6 +21,8 @@ MI_MAX_SLOTS = 128
 MAX_DECODE_TOKENS = 16
 MI_I8_ROW_SCALES = 0         # s [n_in]: the reference's per-row scales [in, 1]
 MI_I8_COL_SCALES = 1         # s [n_out]: per-column scales [1, out]
+I8_CTR_BYTES = 2 * 1024 * 128   # counters at the start of every int8 / bf16 streaming workspace
+MI_W_BF16 = 3                # mi_mlp_many: bf16 weights
 MI_I8_COL_AFTER = 2          # s [n_out] applied after the dot (the int8 lm_head)
 MI_I8_TILED = 0x100          # OR'ed into scale_axis: qT in the tiled layout of mi_int8_tile
 MI_COMBINE_MATMUL = 0
@@ -107,6 +109,8 @@ def lib():
         "mi_bf16_project_workspace": (Z, [I, I, I]),
         "mi_bf16_mlp": (I, [P, I, I, I, P, P, P, F, P, P, P, Z, P]),
         "mi_bf16_mlp_workspace": (Z, [I, I, I]),
+        "mi_mlp_many": (I, [P, I, I, I, P, P, P, P, I, P, P, I, F, P, P, P, Z, P]),
+        "mi_mlp_many_workspace": (Z, [I, I, I]),
         "mi_moe_route": (I, [P, P, P, I, I, I, I, I, F, P, P, P, Z, P]),
         "mi_moe_route_workspace": (Z, [I, I, I]),
         "mi_pack_planes": (I, [I, P, I, I, I, ctypes.POINTER(ctypes.c_void_p), P]),

@@ -453,6 +453,12 @@ __global__ void __launch_bounds__(256) int8_tile_kernel(const int8_t *__restrict
     }
 }
 
+}  // namespace mi
+
+#include "dense_gemm.h"
+
+namespace mi {
+
 // LDS bytes of a split of `cols` columns: B staged activation rows at the padded pitch (+ one f32 scale per column
 // with per-input-row scales).
 static size_t i8_lds_bytes(int B, int cols, int scale_axis) {
@@ -624,7 +630,161 @@ static int mlp_launches(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I,
                      0.0f, nullptr);
 }
 
+// ------------------------------------------------------------------------------------------------ many tokens
+// Token tile and column splits of one dense_gemm launch over `rows` weight rows (both tables of a pair).
+//
+// Tiles of 128 tokens reuse a converted weight twice as often as tiles of 64, but halve the workgroups: they pay from
+// about 24 steps of a 128 x 128 tile per CU on (D 6144, I 2048: 512 tokens 76 us against 82, 128 tokens 42 against 39;
+// D 2048, I 768 at 1500 tokens 48 against 45).
+// Splits fill the chip's two workgroups per CU, but every split writes and reads back f32 partials of the whole
+// output: up to 192 workgroups a split pays down to 8 steps each (down, 64 tokens: 32 us with 4 splits, 36 with 2),
+// beyond that only with 24 steps left (gate/up at 512 tokens: 4 splits 76 us, 2 splits 81; down at 512 tokens, 32 steps
+// in all: 1 split 76, 2 splits 79).
+struct DgPlan {
+    int nt16, nt, mt, S;        // token tiles of 16 per wavefront (2 or 4), token tiles, weight tiles, splits
+};
+
+static DgPlan dg_plan(int B, int K, int rows, Knob s_knob) {
+    DgPlan p;
+    p.mt = rows / kDgRows;
+    const int steps = K / kDgCols;
+    p.nt16 = tuning(kTuneDgNt, 0);
+    if (p.nt16 != 2 && p.nt16 != 4) p.nt16 = B > 64 && (long long)p.mt * ((B + 127) / 128) * steps >= 24 * 256 ? 4 : 2;
+    p.nt = (B + 32 * p.nt16 - 1) / (32 * p.nt16);
+    p.S = 1;
+    for (const long long tiles = (long long)p.mt * p.nt; tiles * p.S * 2 <= 512; p.S *= 2) {
+        const int left = steps / (2 * p.S);
+        if (left < (tiles * p.S < 192 ? 8 : 24)) break;
+    }
+    const int forced = tuning(s_knob, 0);
+    if (forced > 0) p.S = std::min(forced, steps);
+    return p;
+}
+
+static int dg_launch(const DgPlan &p, int form, bool pair, DgArgs a, hipStream_t s) {
+    a.nt = p.nt;
+    a.mt = p.mt;
+    a.S = p.S;
+    typedef void (*Kern)(DgArgs);
+    static const Kern kern[2][2][4] = {
+        {{dense_gemm_kernel<0, false, 2>, dense_gemm_kernel<1, false, 2>, nullptr, dense_gemm_kernel<kW16, false, 2>},
+         {dense_gemm_kernel<0, false, 4>, dense_gemm_kernel<1, false, 4>, nullptr, dense_gemm_kernel<kW16, false, 4>}},
+        {{dense_gemm_kernel<0, true, 2>, dense_gemm_kernel<1, true, 2>, nullptr, dense_gemm_kernel<kW16, true, 2>},
+         {dense_gemm_kernel<0, true, 4>, dense_gemm_kernel<1, true, 4>, nullptr, dense_gemm_kernel<kW16, true, 4>}}};
+    const int groups = (p.mt * p.S + 7) / 8 * 8;       // whole XCD rounds
+    hipLaunchKernelGGL(kern[pair][p.nt16 == 4][form], dim3(groups * p.nt), dim3(256), 0, s, a);
+    return hipGetLastError() == hipSuccess ? MI_OK : MI_ERR_LAUNCH;
+}
+
+// Workspace of mi_mlp_many: [gate partials][up partials][h][down partials].
+struct DgLayout {
+    DgPlan gu, dn;
+    size_t off_u, off_h, off_d, total;
+};
+
+static bool dg_layout(int B, int D, int I, DgLayout &L) {
+    // every 32-bit byte offset of the launches (a token tile of x or h, a table's rows) and every element count of
+    // the sum kernels (B times n_out, in int) stays below 2^31
+    if (B <= 0 || B > (1 << 14) || D <= 0 || I <= 0 || D % 256 || I % 256 || D > 65536 || I > 65536 ||
+        (long long)D * I >= (1ll << 31))
+        return false;
+    L.gu = dg_plan(B, D, 2 * I, kTuneDgS1);
+    L.dn = dg_plan(B, I, D, kTuneDgS2);
+    const size_t gp = L.gu.S > 1 ? al256_i8(4 * (size_t)L.gu.S * B * I) : 0;
+    L.off_u = gp;
+    L.off_h = 2 * gp;
+    L.off_d = L.off_h + al256_i8(2 * (size_t)B * I);
+    L.total = L.off_d + (L.dn.S > 1 ? 4 * (size_t)L.dn.S * B * D : 0);
+    return true;
+}
+
 extern "C" {
+
+size_t mi_mlp_many_workspace(int32_t B, int32_t D, int32_t I) {
+    DgLayout L;
+    return dg_layout(B, D, I, L) ? L.total : 0;
+}
+
+int mi_mlp_many(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I, const void *gate_w, const float *gate_s,
+                const void *up_w, const float *up_s, int32_t gu_form, const void *down_w, const float *down_s,
+                int32_t down_form, float limit, uint16_t *y_bf16, float *y_f32, void *workspace,
+                size_t workspace_bytes, void *stream) {
+    const int gf = gu_form & ~MI_I8_TILED, df = down_form & ~MI_I8_TILED;
+    if (!x_bf16 || !gate_w || !up_w || !down_w || (!y_bf16 && !y_f32)) return MI_ERR_NULL;
+    for (const int32_t f : {gu_form, down_form})
+        if (f != MI_I8_ROW_SCALES && f != MI_I8_COL_SCALES && f != (MI_I8_ROW_SCALES | MI_I8_TILED) &&
+            f != (MI_I8_COL_SCALES | MI_I8_TILED) && f != MI_W_BF16)
+            return MI_ERR_ARG;
+    if ((gf != MI_W_BF16 && (!gate_s || !up_s)) || (df != MI_W_BF16 && !down_s)) return MI_ERR_NULL;
+    if (B <= 0 || B > (1 << 14)) return MI_ERR_TOKENS;
+    if (!(limit > 0.0f)) return MI_ERR_ARG;
+    DgLayout L;
+    if (!dg_layout(B, D, I, L)) return MI_ERR_SHAPE;
+    for (const void *p : {(const void *)x_bf16, gate_w, up_w, down_w, (const void *)y_f32, (const void *)workspace})
+        if ((uintptr_t)p % 16) return MI_ERR_ARG;
+    if ((uintptr_t)y_bf16 % 8) return MI_ERR_ARG;
+    if (gf == MI_I8_ROW_SCALES && ((uintptr_t)gate_s % 16 || (uintptr_t)up_s % 16)) return MI_ERR_ARG;
+    if (df == MI_I8_ROW_SCALES && (uintptr_t)down_s % 16) return MI_ERR_ARG;
+    if (!workspace || workspace_bytes < L.total) return MI_ERR_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
+    char *ws = (char *)workspace;
+    uint16_t *h = (uint16_t *)(ws + L.off_h);
+    DgArgs a{};
+    a.x = x_bf16;
+    a.B = B;
+    a.K = D;
+    a.n_out = I;
+    a.w[0] = (const int8_t *)gate_w;
+    a.w[1] = (const int8_t *)up_w;
+    a.s[0] = gate_s;
+    a.s[1] = up_s;
+    a.tiled = (gu_form & MI_I8_TILED) != 0;
+    a.limit = limit;
+    a.h = h;
+    a.part[0] = (float *)ws;
+    a.part[1] = (float *)(ws + L.off_u);
+    int st = dg_launch(L.gu, gf, true, a, s);
+    if (st) return st;
+    if (L.gu.S > 1) {
+        I8Args r{};
+        r.B = B;
+        r.S = L.gu.S;
+        r.limit = limit;
+        r.h = h;
+        for (int j = 0; j < 2; ++j) {
+            r.p[j].n_out = I;
+            r.p[j].part = a.part[j];
+        }
+        hipLaunchKernelGGL(swiglu_pair_i8, dim3((B * (I / 4) + 255) / 256), dim3(256), 0, s, r);
+        if (hipGetLastError() != hipSuccess) return MI_ERR_LAUNCH;
+    }
+    DgArgs d{};
+    d.x = h;
+    d.B = B;
+    d.K = I;
+    d.n_out = D;
+    d.w[0] = d.w[1] = (const int8_t *)down_w;
+    d.s[0] = d.s[1] = down_s;
+    d.tiled = (down_form & MI_I8_TILED) != 0;
+    d.y_bf16 = y_bf16;
+    d.y_f32 = y_f32;
+    d.part[0] = d.part[1] = (float *)(ws + L.off_d);
+    if ((st = dg_launch(L.dn, df, false, d, s))) return st;
+    if (L.dn.S > 1) {
+        I8Args r{};
+        r.B = B;
+        r.S = L.dn.S;
+        r.n_proj = 1;
+        r.scale_axis = df;
+        r.p[0].n_out = D;
+        r.p[0].part = d.part[0];
+        r.p[0].y_bf16 = y_bf16;
+        r.p[0].y_f32 = y_f32;
+        hipLaunchKernelGGL(split_reduce_i8, dim3((B * (D / 4) + 255) / 256), dim3(256), 0, s, r);
+        if (hipGetLastError() != hipSuccess) return MI_ERR_LAUNCH;
+    }
+    return MI_OK;
+}
 
 size_t mi_int8_project_many_workspace(int32_t B, int32_t n_in, const int32_t *n_out, int32_t n_proj,
                                       int32_t scale_axis) {

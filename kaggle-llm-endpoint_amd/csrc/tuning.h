@@ -16,6 +16,7 @@ enum Knob : int {
     kTuneCS1, kTuneCS1Rtw, kTuneCS2, kTuneCS2Rtw,               // CU-balanced one-token launches
     kTuneCustream, kTuneCumulti, kTunePersistAbove, kTuneFuseSwiglu, kTuneCuFormH, kTuneSpinLimit, kTuneCuCombine,
     kTuneI8S, kTuneI8Waves, kTuneI8Fuse,
+    kTuneDgS1, kTuneDgS2, kTuneDgNt,         // many-token MLP: gate/up and down splits, token tiles per wavefront
     kTuneCount
 };
 

@@ -611,6 +611,38 @@ def int8_project_many(x, projections, want_f32=False, outputs=None, workspace=No
     return outs
 
 
+_MLP_MANY_STEP = 4096           # tokens per mi_mlp_many call: bounds its workspace (h, split partials)
+
+
+def _mlp_many(x, ws3, scales, gu_form, down_form, D, I, limit, yb, yf, workspace):
+    """More tokens than one streaming call takes (32), as dense GEMMs (mi_mlp_many).  False, with nothing done, when
+    the call does not fit them: a pointer off its 16-byte alignment (a view into another tensor), or a caller's
+    workspace sized for the 32-token calls."""
+    B = x.shape[0]
+    need = lib().mi_mlp_many_workspace(min(B, _MLP_MANY_STEP), D, I) if B > 32 else 0
+    if need == 0:
+        return False
+    ptrs = [x, yf] + list(ws3) + [s for s in scales if s is not None]
+    if any(t is not None and t.data_ptr() % 16 for t in ptrs) or yb.data_ptr() % 8:
+        return False
+    ws = workspace
+    if ws is not None:
+        # a kept workspace opens with the streaming calls' zero counters: the scratch goes behind them
+        ws = ws[_lib.I8_CTR_BYTES:]
+        if ws.numel() < need or ws.data_ptr() % 16:
+            return False
+    else:
+        ws = WORKSPACES.get("mlp_many", need)
+    for b0 in range(0, B, _MLP_MANY_STEP):
+        n = min(_MLP_MANY_STEP, B - b0)
+        check("mi_mlp_many", lib().mi_mlp_many(_ptr(x[b0:]), n, D, I, _ptr(ws3[0]), _ptr(scales[0]), _ptr(ws3[1]),
+                                               _ptr(scales[1]), int(gu_form), _ptr(ws3[2]), _ptr(scales[2]),
+                                               int(down_form), float(limit), _ptr(yb[b0:]),
+                                               _ptr(yf[b0:]) if yf is not None else None, _ptr(ws), ws.numel(),
+                                               _stream()))
+    return True
+
+
 def int8_mlp(x, gate, up, down, limit, want_f32=False, y_bf16=None, y_f32=None, workspace=None):
     """mlp_partial over int8 leaves (model.py:125-127 with quant8.py:91-99): y = bf16(h @ Wd) with
     h = bf16(swiglu_clamped(bf16(x @ Wg), bf16(x @ Wu))), W = bf16(f32(q) * s).  x bf16 [B, D]; gate, up, down:
@@ -630,6 +662,9 @@ def int8_mlp(x, gate, up, down, limit, want_f32=False, y_bf16=None, y_f32=None, 
     yb = y_bf16 if y_bf16 is not None else torch.empty((B, D), dtype=torch.bfloat16, device=x.device)
     yf = y_f32 if y_f32 is not None else (
         torch.empty((B, D), dtype=torch.float32, device=x.device) if want_f32 else None)
+    if _mlp_many(x, (g[0], u[0], d[0]), (g[1], u[1], d[1]), int(g[2]) | gt, int(d[2]) | dt, D, I, limit, yb, yf,
+                 workspace):
+        return (yb, yf) if want_f32 else yb
     for b0 in range(0, B, 32):
         n = min(32, B - b0)
         nbytes = lib().mi_int8_mlp_workspace(n, D, I, int(g[2]), int(d[2]))
@@ -705,6 +740,8 @@ def bf16_mlp(x, gate, up, down, limit, want_f32=False, y_bf16=None, y_f32=None, 
     yb = y_bf16 if y_bf16 is not None else torch.empty((B, D), dtype=torch.bfloat16, device=x.device)
     yf = y_f32 if y_f32 is not None else (
         torch.empty((B, D), dtype=torch.float32, device=x.device) if want_f32 else None)
+    if _mlp_many(x, (g, u, d), (None, None, None), _lib.MI_W_BF16, _lib.MI_W_BF16, D, I, limit, yb, yf, workspace):
+        return (yb, yf) if want_f32 else yb
     for b0 in range(0, B, 32):
         n = min(32, B - b0)
         nbytes = lib().mi_bf16_mlp_workspace(n, D, I)
