@@ -150,15 +150,9 @@ __device__ __forceinline__ void pf_ctile(const Cb3Wave &w, PfRegs &s, int st, co
 struct PfShared {
     union {
         uint4 cbl[kPfWaves * 5 * 64];            // CB3: per-wavefront codebook slots (20 KB)
-        struct {
-            float4 grid[512];                    // IQ3_S: the grid's levels as f32 (8 KB)
-            uint4 smask[256];                    // IQ3_S: 8 sign bits -> sign bits of 4 bf16 pairs (4 KB)
-        } iq;
-        float2 iq4pair[256];                     // IQ4_XS: byte -> (level of its low nibble, of its high nibble)
-        struct {
-            uint4 level[1024];                   // IQ2_S: grid entry -> its 8 levels as bf16 (16 KB)
-            uint4 smask[256];                    // IQ2_S: 8 sign bits -> sign bits of 4 bf16 pairs (4 KB)
-        } iq2;
+        uint2 iq3grid[512];                      // IQ3_S: grid entry -> its 4 levels as f16 (4 KB)
+        uint32_t iq4pair[256];                   // IQ4_XS: byte -> f16 levels of its low and its high nibble (1 KB)
+        uint2 iq2code[1024];                     // IQ2_S: grid entry -> its 8 levels as codes 0..2, one byte each (8 KB)
     };
     uint32_t xs[2][kPfTm * kPfXPitch];           // column tiles ct (even/odd) of the block's rows, double-buffered;
                                                  // gate/up epilogue: the gate accumulators of one (gate, up) pair
@@ -167,6 +161,14 @@ struct PfShared {
 };
 
 // ------------------------------------------------------------------------------------------------ weight providers
+// The block formats' decode and its LDS table gathers share a step with the matrix-core work, and with up to 5 token
+// tiles per decoded weight they, not the MFMAs, set the pace.  Per 8 weights (a lane's A operand) the loops issue
+// (vector instructions / table gathers, before -> now): IQ2_S 44 / 2 x 16 bytes -> 25 / 8 bytes (levels through a
+// byte-permute table of the three scaled levels and their negatives), IQ3_S 41 / 3 x 16 -> 31 / 2 x 8, IQ4_XS 35 /
+// 4 x 8 -> 23 / 4 x 4 (f16 levels widened inside the multiply), Q2_K 48 -> 27 (byte-permute table).  Measured at
+// D 6144, I 2048, 64 experts, top-8, same bits: IQ2_S + IQ4_XS 27 tokens 453 -> 330 us, 512 tokens 705 -> 577, IQ3_S
+// 1999 tokens 2288 -> 1919.
+//
 // A provider streams the weights of one wavefront's 64 rows (4 row tiles) of expert e, one column tile at a time, and
 // runs the tile's k-steps on the matrix cores against the staged activations.  Its state is two values the workgroup
 // body keeps as locals: Wave (addressing, fixed per wavefront) and Regs (the loads in flight).
@@ -230,8 +232,23 @@ struct PfCb3 {
 constexpr int kIq3TileCols = 128;
 
 __device__ __forceinline__ uint32_t pf_bf16_pair(float a, float b) {   // round to nearest even
-    const __bf16 v[2] = {(__bf16)a, (__bf16)b};
+    // one v_cvt_pk_bf16_f32 (an array of two __bf16 compiles to two conversions, a shift and an or)
+    const bf16x2 v = {(__bf16)a, (__bf16)b};
     return __builtin_bit_cast(uint32_t, v);
+}
+
+// f16 half H (0 low, 1 high) of v times s in f32 (v_fma_mix_f32: the f16 is widened in the instruction).
+template <int H>
+__device__ __forceinline__ float pf_mix(uint32_t v, float s) {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    return fmaf((float)__builtin_bit_cast(f16x2, v)[H], s, 0.0f);
+}
+
+// The 16-bit values at bytes sel[b] of a table of up to 8 entries held as low and high bytes (entries 0..3 in *0, 4..7
+// in *1), for the 4 selector bytes of sel: two dwords of bf16 pairs.
+__device__ __forceinline__ uint2 pf_lookup4(uint32_t lo0, uint32_t lo1, uint32_t hi0, uint32_t hi1, uint32_t sel) {
+    const uint32_t l = perm(lo1, lo0, sel), h = perm(hi1, hi0, sel);
+    return make_uint2(perm(h, l, 0x05010400u), perm(h, l, 0x07030602u));
 }
 
 // One plane word (4 bytes) per lane at base + off if `use`, else zero: a buffer load through a descriptor whose
@@ -250,8 +267,7 @@ struct PfIq3Wave {
     uint32_t lrow;                          // the lane's byte offset in a plane row (row jt of the wavefront)
     int q;                                  // the lane's group
     int CT;                                 // column tiles of a row
-    const float4 *grid;                     // LDS: the grid's levels as f32
-    const uint4 *smask;                     // LDS: sign masks
+    const uint2 *grid;                      // LDS: the grid's levels as f16
 };
 struct PfIq3Regs {
     // plane words of column tile ct in slot ct & 1, per row tile: qs of words q and 4 + q, their sg words, qh, sc, d
@@ -292,8 +308,7 @@ struct PfIq3 {
         w.q = lane >> 4;
         w.lrow = 4u * (uint32_t)(rg * 64 + (lane & 15));
         w.CT = min(tb.K / kIq3TileCols, 4 * st1);          // prefetch no column tile past the range
-        w.grid = sh.iq.grid;
-        w.smask = sh.iq.smask;
+        w.grid = sh.iq3grid;
         (void)wave;
 #pragma unroll
         for (int c = 0; c < 2; ++c)
@@ -304,19 +319,21 @@ struct PfIq3 {
     static __device__ __forceinline__ bf16x8 weights8(const Wave &w, const uint32_t (&u)[7], int ct, int j) {
         const int m = j >> 1, half = j & 1, q = w.q;
         const uint32_t word = m ? u[1] : u[0];
-        const uint32_t s8 = ((m ? u[3] : u[2]) >> (16 * (q & 1) + 8 * half)) & 255u;
-        const uint32_t qh4 = (u[4] >> (4 * (4 * m + q))) & 15u;
-        const uint32_t nib = (u[5] >> (4 * (4 * (ct & 1) + 2 * m + (q >> 1)))) & 15u;
+        // the word's 16 signs; sg2 has sign 2p at bit 2p and sign 2p + 1 at bit 2p + 16, a pair's two bf16 sign
+        // bits once shifted left by 15 - 2p
+        const uint32_t sg = ((m ? u[3] : u[2]) >> (16 * (q & 1))) & 0xffffu, sg2 = (sg << 15) | sg;
+        const uint32_t qh4 = u[4] >> (4 * q) >> (16 * m);
+        const uint32_t nib = (u[5] >> (4 * (q >> 1)) >> (16 * (ct & 1) + 8 * m)) & 15u;
         const float scale = f16_bits_to_f32(u[6] >> (16 * ((ct >> 1) & 1))) * (float)(1u + 2u * nib);
         const uint32_t i0 = ((word >> (16 * half)) & 255u) | (((qh4 >> (2 * half)) & 1u) << 8);
         const uint32_t i1 = ((word >> (16 * half + 8)) & 255u) | (((qh4 >> (2 * half + 1)) & 1u) << 8);
-        const float4 g0 = w.grid[i0], g1 = w.grid[i1];
-        const uint4 sm = w.smask[s8];
+        const uint2 g0 = w.grid[i0], g1 = w.grid[i1];
+        const int sh = 15 - 8 * half;
         uint4 A;
-        A.x = pf_bf16_pair(g0.x * scale, g0.y * scale) | sm.x;
-        A.y = pf_bf16_pair(g0.z * scale, g0.w * scale) | sm.y;
-        A.z = pf_bf16_pair(g1.x * scale, g1.y * scale) | sm.z;
-        A.w = pf_bf16_pair(g1.z * scale, g1.w * scale) | sm.w;
+        A.x = pf_bf16_pair(pf_mix<0>(g0.x, scale), pf_mix<1>(g0.x, scale)) ^ ((sg2 << sh) & 0x80008000u);
+        A.y = pf_bf16_pair(pf_mix<0>(g0.y, scale), pf_mix<1>(g0.y, scale)) ^ ((sg2 << (sh - 2)) & 0x80008000u);
+        A.z = pf_bf16_pair(pf_mix<0>(g1.x, scale), pf_mix<1>(g1.x, scale)) ^ ((sg2 << (sh - 4)) & 0x80008000u);
+        A.w = pf_bf16_pair(pf_mix<0>(g1.y, scale), pf_mix<1>(g1.y, scale)) ^ ((sg2 << (sh - 6)) & 0x80008000u);
         return __builtin_bit_cast(bf16x8, A);
     }
     template <int NTT, int C>
@@ -357,8 +374,7 @@ struct PfIq2Wave {
     uint32_t rpitch;                        // bytes per plane row (4 R)
     uint32_t lrow;                          // the lane's byte offset in a plane row (row jt of the wavefront)
     int q, CT;
-    const uint4 *level;                     // LDS: grid entry -> 8 bf16 levels
-    const uint4 *smask;                     // LDS: sign masks
+    const uint2 *code;                      // LDS: grid entry -> 8 level codes
 };
 struct PfIq2Regs {
     uint32_t v[2][kPfRtw][5];   // column tile ct in slot ct & 1, per row tile: the lane's qs and sg words, qh, sc, d
@@ -393,45 +409,58 @@ struct PfIq2 {
         w.q = lane >> 4;
         w.lrow = 4u * (uint32_t)(rg * 64 + (lane & 15));
         w.CT = min(tb.K / 128, 4 * st1);                   // prefetch no column tile past the range
-        w.level = sh.iq2.level;
-        w.smask = sh.iq2.smask;
+        w.code = sh.iq2code;
         (void)wave;
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
             for (int r = 0; r < kPfRtw; ++r) load(w, 4 * st0 + c, s.v[c][r], r, true);
     }
+    // The scaled levels of one 16-weight scale group as a byte table: entry c (0..2) is bf16(level c * scale), entry
+    // c + 4 its negative; low bytes, high bytes, high bytes of the negatives.
+    struct Levels {
+        uint32_t lo, hi, neg;
+    };
+    static __device__ __forceinline__ Levels levels(const Wave &w, const uint32_t (&u)[5], int ct, int jj) {
+        const uint32_t nib = (u[3] >> (8 * w.q) >> (4 * jj)) & 15u;
+        const float scale = f16_bits_to_f32(u[4] >> (16 * ((ct >> 1) & 1))) * 0.25f * (0.5f + (float)nib);
+        const uint32_t c01 = pf_bf16_pair(8.0f * scale, 25.0f * scale), c2 = pf_bf16_pair(43.0f * scale, 0.0f);
+        Levels t;
+        t.lo = perm(c2, c01, 0x0c040200u);
+        t.hi = perm(c2, c01, 0x0c050301u);
+        t.neg = t.hi ^ 0x80808080u;
+        return t;
+    }
     // the 8 weights of step j (group j of the lane's word) for the row tile whose plane words are u
-    static __device__ __forceinline__ bf16x8 weights8(const Wave &w, const uint32_t (&u)[5], int ct, int j) {
-        const int q = w.q;
-        const uint32_t idx = ((u[0] >> (8 * j)) & 255u) | (((u[2] >> (8 * q + 2 * j)) & 3u) << 8);
-        const uint32_t s8 = (u[1] >> (8 * j)) & 255u;
-        const uint32_t nib = (u[3] >> (8 * q + 4 * (j >> 1))) & 15u;
-        const float scale = f16_bits_to_f32(u[4] >> (16 * ((ct >> 1) & 1))) * (0.5f + (float)nib) * 0.25f;
-        const uint4 g = w.level[idx];
-        const uint4 sm = w.smask[s8];
-        uint4 A;
-        A.x = pf_bf16_pair(__uint_as_float(g.x << 16) * scale, __uint_as_float(g.x & 0xffff0000u) * scale) | sm.x;
-        A.y = pf_bf16_pair(__uint_as_float(g.y << 16) * scale, __uint_as_float(g.y & 0xffff0000u) * scale) | sm.y;
-        A.z = pf_bf16_pair(__uint_as_float(g.z << 16) * scale, __uint_as_float(g.z & 0xffff0000u) * scale) | sm.z;
-        A.w = pf_bf16_pair(__uint_as_float(g.w << 16) * scale, __uint_as_float(g.w & 0xffff0000u) * scale) | sm.w;
-        return __builtin_bit_cast(bf16x8, A);
+    static __device__ __forceinline__ bf16x8 weights8(const Wave &w, const uint32_t (&u)[5], const Levels &t, int j) {
+        const uint32_t idx = ((u[0] >> (8 * j)) & 255u) | (((u[2] >> (8 * w.q) >> (2 * j)) & 3u) << 8);
+        const uint2 c = w.code[idx];
+        // 4 sign bits to bit 2 of 4 bytes: one 24-bit multiply (shifts by 2, 9, 16, 23: no two bits meet)
+        const uint32_t s0 = __umul24((u[1] >> (8 * j)) & 15u, 0x810204u) & 0x04040404u;
+        const uint32_t s1 = __umul24((u[1] >> (8 * j + 4)) & 15u, 0x810204u) & 0x04040404u;
+        const uint2 a0 = pf_lookup4(t.lo, t.lo, t.hi, t.neg, c.x | s0), a1 = pf_lookup4(t.lo, t.lo, t.hi, t.neg, c.y | s1);
+        return __builtin_bit_cast(bf16x8, make_uint4(a0.x, a0.y, a1.x, a1.y));
     }
     template <int NTT, int C>
     static __device__ __forceinline__ void tile(const Wave &w, Regs &s, int st, const uint32_t *xt,
                                                 f32x4 (&acc)[kPfRtw][NTT]) {
         const int ct = 4 * st + C;
+        Levels lv[kPfRtw];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if (j > 0) __builtin_amdgcn_sched_barrier(0);
             uint4 b[NTT];
 #pragma unroll
             for (int tt = 0; tt < NTT; ++tt) b[tt] = *(const uint4 *)(xt + tt * 16 * kPfXPitch + 4 * j);
-            bf16x8 A = weights8(w, s.v[C & 1][0], ct, j);
+            if ((j & 1) == 0) lv[0] = levels(w, s.v[C & 1][0], ct, j >> 1);
+            bf16x8 A = weights8(w, s.v[C & 1][0], lv[0], j);
 #pragma unroll
             for (int r = 0; r < kPfRtw; ++r) {
                 bf16x8 An = A;
-                if (r + 1 < kPfRtw) An = weights8(w, s.v[C & 1][r + 1], ct, j);
+                if (r + 1 < kPfRtw) {
+                    if ((j & 1) == 0) lv[r + 1] = levels(w, s.v[C & 1][r + 1], ct, j >> 1);
+                    An = weights8(w, s.v[C & 1][r + 1], lv[r + 1], j);
+                }
 #pragma unroll
                 for (int tt = 0; tt < NTT; ++tt) acc[r][tt] = mfma16(A, b[tt], acc[r][tt]);
                 A = An;
@@ -520,8 +549,13 @@ struct PfKq {
             m = d * ((float)sb - 32.0f);                              // exact
             a = -4.0f * m;
         } else {
+            // the scale group's four values as a byte table: v = 0..3 -> bf16(v * m + a)
             m = d * (float)(sb & 15u);
             a = -(f16_bits_to_f32(u[4] >> 16) * (float)(sb >> 4));
+            const uint32_t c01 = pf_bf16_pair(a, m + a), c23 = pf_bf16_pair(fmaf(2.0f, m, a), fmaf(3.0f, m, a));
+            const uint32_t lo = perm(c23, c01, 0x06040200u), hi = perm(c23, c01, 0x07050301u);
+            const uint2 l0 = pf_lookup4(lo, lo, hi, hi, t0), l1 = pf_lookup4(lo, lo, hi, hi, t1);
+            return __builtin_bit_cast(bf16x8, make_uint4(l0.x, l0.y, l1.x, l1.y));
         }
         const uint2 l0 = four(t0, m, a), l1 = four(t1, m, a);
         return __builtin_bit_cast(bf16x8, make_uint4(l0.x, l0.y, l1.x, l1.y));
@@ -563,7 +597,7 @@ struct PfIq4Wave {
     uint32_t rpitch;                        // bytes per plane row (4 R)
     uint32_t lrow;                          // the lane's byte offset in a plane row (row jt of the wavefront)
     int q, CT;
-    const float2 *pair;                     // LDS: byte -> its two levels as f32
+    const uint32_t *pair;                   // LDS: byte -> its two levels as f16
 };
 struct PfIq4Regs {
     uint32_t v[2][kPfRtw][7];   // column tile ct in slot ct & 1, per row tile: the 4 words, sl, sh, d
@@ -610,13 +644,13 @@ struct PfIq4 {
         const int sv = (int)(((u[4] >> (4 * i)) & 15u) | (((u[5] >> (2 * i)) & 3u) << 4)) - 32;
         const float scale = f16_bits_to_f32(u[6] >> (16 * ((ct >> 1) & 1))) * (float)sv;
         const uint32_t x = u[j];
-        const float2 p0 = w.pair[x & 255u], p1 = w.pair[(x >> 8) & 255u], p2 = w.pair[(x >> 16) & 255u],
-                     p3 = w.pair[x >> 24];
+        const uint32_t p0 = w.pair[x & 255u], p1 = w.pair[(x >> 8) & 255u], p2 = w.pair[(x >> 16) & 255u],
+                       p3 = w.pair[x >> 24];
         uint4 A;
-        A.x = pf_bf16_pair(p0.x * scale, p1.x * scale);
-        A.y = pf_bf16_pair(p2.x * scale, p3.x * scale);
-        A.z = pf_bf16_pair(p0.y * scale, p1.y * scale);
-        A.w = pf_bf16_pair(p2.y * scale, p3.y * scale);
+        A.x = pf_bf16_pair(pf_mix<0>(p0, scale), pf_mix<0>(p1, scale));
+        A.y = pf_bf16_pair(pf_mix<0>(p2, scale), pf_mix<0>(p3, scale));
+        A.z = pf_bf16_pair(pf_mix<1>(p0, scale), pf_mix<1>(p1, scale));
+        A.w = pf_bf16_pair(pf_mix<1>(p2, scale), pf_mix<1>(p3, scale));
         return __builtin_bit_cast(bf16x8, A);
     }
     template <int NTT, int C>
@@ -898,46 +932,26 @@ __global__ void __launch_bounds__(64 * kPfWaves, 2) prefill_kernel(PfArgs a) {
     }
     const int e = __builtin_amdgcn_readfirstlane(a.blk_expert[g]);
     const int n = __builtin_amdgcn_readfirstlane(a.blk_n[g]);
+    // the format's LDS table (published by the barrier after the row offsets)
+    const auto f16_pair = [](float lo, float hi) {
+        return (uint32_t)__builtin_bit_cast(unsigned short, (_Float16)lo) |
+               (uint32_t)__builtin_bit_cast(unsigned short, (_Float16)hi) << 16;
+    };
     if constexpr (std::is_same<WP, PfIq3>::value) {
-        // the grid's levels as f32 and the sign masks (published by the barrier after the row offsets)
-        const int tid = threadIdx.x;
-        for (int i = tid; i < 512; i += 64 * kPfWaves) {
+        for (int i = threadIdx.x; i < 512; i += 64 * kPfWaves) {
             const uint32_t v = kPfGrid[i];
-            sh.iq.grid[i] = make_float4((float)(v & 255u), (float)((v >> 8) & 255u), (float)((v >> 16) & 255u),
-                                        (float)(v >> 24));
-        }
-        if (tid < 256) {
-            uint32_t m[4];
-#pragma unroll
-            for (int p = 0; p < 4; ++p) m[p] = (((uint32_t)tid >> (2 * p)) & 1u) << 15 | (((uint32_t)tid >> (2 * p + 1)) & 1u) << 31;
-            sh.iq.smask[tid] = make_uint4(m[0], m[1], m[2], m[3]);
+            sh.iq3grid[i] = make_uint2(f16_pair((float)(v & 255u), (float)((v >> 8) & 255u)),
+                                       f16_pair((float)((v >> 16) & 255u), (float)(v >> 24)));
         }
     }
     if constexpr (std::is_same<WP, PfIq2>::value) {
-        // the grid's levels as bf16 and the sign masks (published by the barrier after the row offsets)
-        const int tid = threadIdx.x;
-        for (int i = tid; i < 1024; i += 64 * kPfWaves) {
-            const uint32_t lo = kPfGrid2[2 * i], hi = kPfGrid2[2 * i + 1];
-            uint32_t v[4];
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const uint32_t wd = p < 2 ? lo : hi, sft = 16 * (p & 1);
-                v[p] = (__float_as_uint((float)((wd >> sft) & 255u)) >> 16) |
-                       (__float_as_uint((float)((wd >> (sft + 8)) & 255u)) & 0xffff0000u);
-            }
-            sh.iq2.level[i] = make_uint4(v[0], v[1], v[2], v[3]);
-        }
-        if (tid < 256) {
-            uint32_t m[4];
-#pragma unroll
-            for (int p = 0; p < 4; ++p) m[p] = (((uint32_t)tid >> (2 * p)) & 1u) << 15 | (((uint32_t)tid >> (2 * p + 1)) & 1u) << 31;
-            sh.iq2.smask[tid] = make_uint4(m[0], m[1], m[2], m[3]);
-        }
+        // levels 8, 25, 43 -> codes 0, 1, 2
+        for (int i = threadIdx.x; i < 1024; i += 64 * kPfWaves)
+            sh.iq2code[i] = make_uint2((kPfGrid2[2 * i] >> 4) & 0x03030303u, (kPfGrid2[2 * i + 1] >> 4) & 0x03030303u);
     }
     if constexpr (std::is_same<WP, PfIq4>::value) {
-        // the level pairs (published by the barrier after the row offsets)
         for (int i = threadIdx.x; i < 256; i += 64 * kPfWaves)
-            sh.iq4pair[i] = make_float2((float)kPfKv[i & 15], (float)kPfKv[i >> 4]);
+            sh.iq4pair[i] = f16_pair((float)kPfKv[i & 15], (float)kPfKv[i >> 4]);
     }
     switch ((n + 15) >> 4) {
         case 1: prefill_body<MODE, 1, WP, FORM>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
