@@ -29,6 +29,7 @@ struct PlanOut {
     float *w_row;          // [Rp]  routing weight of every sorted row, 0 = padding
     int32_t *row_slot;     // [T * kk] sorted row of every (token, slot); -1 for an expert id outside [0, E)
     int32_t *blk_n;        // [G]   rows of every block that are not padding (NULL: not written)
+    int32_t *blk_order;    // [G]   blocks in launch order: most token tiles first (NULL: not written)
     int merge_dups;        // w_row of the first slot of a token's expert = the sum of that token's weights of the
                            // expert in column order, 0 for its later slots (the sweeps' summed routing weight)
     uint32_t *cnt;         // [n_cnt] the grouped GEMMs' split-task counters, zeroed here (NULL: none)
@@ -102,6 +103,7 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
     __shared__ int cnt[kPlanMaxE], bend[kPlanMaxE], rbase[kPlanMaxE];
     __shared__ unsigned long long lanes[kPlanWaves][kPlanMaskE];   // pass 2: lanes of every id in this step
     __shared__ int wsum[kPlanWaves];
+    __shared__ int ntile[kPfTT + 1];              // blocks of every token tile count, then the first position of each
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kk = k + (shared >= 0 ? 1 : 0);
     const int S = T * kk;
@@ -189,6 +191,7 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
     __syncthreads();
     const int n_blocks = bend[kPlanMaxE - 1];
     if (tid == 0) *p.n_blocks = n_blocks;
+    if (tid <= kPfTT) ntile[tid] = 0;
     for (int i = tid; i < p.n_cnt; i += kPlanThreads) p.cnt[i] = 0u;
     vm_wait<0>();                              // this wavefront's padding stores are done ...
     __syncthreads();                            // ... and every other wavefront's
@@ -255,7 +258,23 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
         }
         p.blk_expert[g] = e;
         if (p.blk_n) p.blk_n[g] = n;
+        if (p.blk_order && n > 0) atomicAdd(&ntile[(n + 15) >> 4], 1);
     }
+    if (!p.blk_order) return;
+    // launch order: a counting sort by token tiles, most first, so the launches' last tasks are their shortest (the
+    // order among equals is free: it changes no result)
+    vm_wait<0>();                                 // blk_n as stored above
+    __syncthreads();
+    if (tid == 0) {
+        int at = 0;
+        for (int c = kPfTT; c > 0; --c) {
+            const int m = ntile[c];
+            ntile[c] = at;
+            at += m;
+        }
+    }
+    __syncthreads();
+    for (int g = tid; g < n_blocks; g += kPlanThreads) p.blk_order[atomicAdd(&ntile[(p.blk_n[g] + 15) >> 4], 1)] = g;
 }
 
 // out[t] = sum_j wt(t, j) * y[row_slot(t, j)] over the plan's kk columns in order, f32; wt = bf16(w) for the matmul
@@ -381,11 +400,11 @@ __global__ void __launch_bounds__(256) prefill_combine_f32(const float *__restri
 struct PfLayout {
     int S, G, P;
     long long Rp;
-    size_t off_be, off_nb, off_bn, off_tr, off_wr, off_rs, off_h, off_y, off_part, off_cnt, total;
+    size_t off_be, off_nb, off_bn, off_bo, off_tr, off_wr, off_rs, off_h, off_y, off_part, off_cnt, total;
 };
 
-// Workgroups of a grouped GEMM launch resident at once: 2 per CU (the 77 KB of LDS and <= 256 VGPRs per wavefront
-// of prefill_kernel).  The launches split their last round's tasks by it (prefill_gemm.h).
+// Workgroups of a block-format GEMM launch resident at once: kPfBPerSimd per CU, one wavefront of each on every SIMD.
+// The launches split their last round's tasks by it (prefill_gemm.h).
 static int pf_slots() {
     static int slots = 0;
     if (!slots) {
@@ -393,7 +412,7 @@ static int pf_slots() {
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
             cus = 256;
-        slots = 2 * cus;
+        slots = kPfBPerSimd * cus;
     }
     return slots;
 }
@@ -412,6 +431,7 @@ static PfLayout pf_layout(int T, int kk, int E, int I, int D, bool y32) {
     L.off_be = o; o = al256(o + 4 * (size_t)L.G);
     L.off_nb = o; o = al256(o + 4);
     L.off_bn = o; o = al256(o + 4 * (size_t)L.G);
+    L.off_bo = o; o = al256(o + 4 * (size_t)L.G);
     L.off_tr = o; o = al256(o + 4 * (size_t)L.Rp);
     L.off_wr = o; o = al256(o + 4 * (size_t)L.Rp);
     L.off_rs = o; o = al256(o + 4 * (size_t)L.S);
@@ -547,7 +567,7 @@ int mi_ragged_plan(const int32_t *idx, const float *w, int32_t T, int32_t k, int
     if (T <= 0 || k <= 0) return MI_ERR_TOKENS;
     if (E <= 0 || E > kPlanMaxE || tm <= 0 || tm > 65536) return MI_ERR_ARG;
     if (!plan_sizes_ok(T, k, E, tm)) return MI_ERR_TOKENS;
-    PlanOut p{blk_expert, n_blocks, tok_row, w_row, row_slot, nullptr, 0, nullptr, 0};
+    PlanOut p{blk_expert, n_blocks, tok_row, w_row, row_slot, nullptr, nullptr, 0, nullptr, 0};
     return launch_plan(idx, w, T, k, -1, E, tm, p, (hipStream_t)stream);
 }
 
@@ -598,6 +618,7 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     p.blk_expert = (int32_t *)(ws + L.off_be);
     p.n_blocks = (int32_t *)(ws + L.off_nb);
     p.blk_n = (int32_t *)(ws + L.off_bn);
+    p.blk_order = (int32_t *)(ws + L.off_bo);
     p.tok_row = (int32_t *)(ws + L.off_tr);
     p.w_row = (float *)(ws + L.off_wr);
     p.row_slot = (int32_t *)(ws + L.off_rs);
@@ -628,6 +649,7 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     a.K = gate->cols;
     a.blk_expert = p.blk_expert;
     a.blk_n = p.blk_n;
+    a.blk_order = p.blk_order;
     a.n_blocks = p.n_blocks;
     a.tok_row = p.tok_row;
     a.x = x_bf16;
@@ -635,13 +657,12 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     a.gather = 1;
     a.out = h;
     a.limit = limit;
-    a.wg_rows = 2;
-    a.RBG = I / 128;
+    a.RBG = gate->qtype == MI_QT_CB3 ? I / 128 : I / (8 * kPfBWaves * kPfBRtw);
     a.w_row = p.w_row;
     a.P = L.P;
     a.part = (float *)(ws + L.off_part);
     a.cnt = p.cnt;
-    // blocks rounded up to whole XCD rounds, then the split tasks' pieces (at most P)
+    // every block's tasks and at most P pieces of split ones, in whole XCD rounds
     const int g8 = (L.G + kXcds - 1) / kXcds * kXcds;
     const bool round_gu = combine == MI_COMBINE_XLA_GATHER || combine == MI_COMBINE_XLA_SWEEP;
     const dim3 ggu(g8 * a.RBG + L.P);
@@ -661,8 +682,7 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     b.x_bytes = (uint32_t)(L.Rp * I * 2);
     b.gather = 0;
     b.out = y;
-    b.wg_rows = 4;
-    b.RBG = D / 256;
+    b.RBG = down->qtype == MI_QT_CB3 ? D / 256 : D / (16 * kPfBWaves * kPfBRtw);
     b.out32 = (float *)y;
     const dim3 gdn(g8 * b.RBG + L.P);
     if ((st = y32 ? launch_prefill_1_4(down->qtype, gdn, s, b) : launch_prefill_1_0(down->qtype, gdn, s, b))) return st;

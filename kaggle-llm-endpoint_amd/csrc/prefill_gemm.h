@@ -2,8 +2,8 @@
 // reference's moe_ragged_gateup / moe_ragged_down, pallas_moe.py:622-755, and the rounding forms of its other bf16
 // prefill branches, resident.py:122-135,169-210):
 //   prefill_kernel<MODE, WP, FORM>  one workgroup per (block, row range) streams the block's expert once for all
-//                       its rows: each wavefront owns 64 weight rows x up to 80 rows of activations (5 MFMA token
-//                       tiles), decodes every weight once (CB3: the decoder of cb3_tiles.h; IQ3_S: the planes straight
+//                       its rows: each wavefront owns 64 (CB3) or 32 weight rows x up to 80 rows of activations (5
+//                       MFMA token tiles), decodes every weight once (CB3: the decoder of cb3_tiles.h; IQ3_S: the planes straight
 //                       into the A operand) and reuses it across the token tiles; the block's activation rows are
 //                       staged one column tile (160 / 128 columns) at a time in LDS;
 //                         gate/up: h = bf16(silu(min(g, L)) * clip(u, -L, L)), g and u f32    (pallas_moe.py:682)
@@ -32,8 +32,13 @@ static __constant__ int8_t kPfKv[16] = {
 
 constexpr int kPfTT = 5;                   // token tiles of 16 rows per block
 constexpr int kPfTm = 16 * kPfTT;          // rows per block of the prefill's own plan
-constexpr int kPfWaves = 4;
-constexpr int kPfRtw = 4;                  // row tiles per wavefront (64 weight rows)
+constexpr int kPfWaves = 4;                // CB3: wavefronts per workgroup ...
+constexpr int kPfRtw = 4;                  // ... and row tiles per wavefront (64 weight rows)
+// The block formats: 128 rows per workgroup, 4 wavefronts of 32 rows in at most 168 registers and 49 KB of LDS, so that
+// three wavefronts per SIMD cover each other's table gathers, barriers and loads.  IQ2_S + IQ4_XS layer, D 6144, I 2048,
+// against two wavefronts of 64 rows (256 registers, 77 KB) with the same decoders: 27 tokens 319 -> 292 us, 512 tokens
+// the same; in launch order by token tiles with the last blocks' tasks dealt singly 285 and 531 (from 541)
+constexpr int kPfBWaves = 4, kPfBRtw = 2, kPfBPerSimd = 3;
 constexpr int kPfXPitch = 88;              // dwords per staged activation row of one column tile (80 + 8: the
                                            // fastest pitch for this read pattern on gfx950, measured)
 constexpr int kPfGPitch = kPfTm + 4;       // floats per row of the gate/up epilogue's exchange (skewed banks)
@@ -48,13 +53,12 @@ struct PfArgs {
     Iq2Table j0, j1;                       // IQ2_S tables, the same roles
     KqTable q0, q1;                        // Q2_K / Q3_K tables, the same roles
     int R, K;                              // output columns (rows of the table), input columns
-    const int32_t *blk_expert, *blk_n, *n_blocks, *tok_row;
+    const int32_t *blk_expert, *blk_n, *blk_order, *n_blocks, *tok_row;
     const uint16_t *x;                     // gate/up: x [T, K] gathered through tok_row; down: h [Rp, K]
     uint32_t x_bytes;                      // bytes of x (< 2^31)
     int gather;
     uint16_t *out;                         // gate/up: h [Rp, R]; down: y [Rp, R]
     float limit;
-    int wg_rows;                           // 64-row groups per workgroup: gate/up 2 (x gate, up), down 4
     int RBG;                               // workgroups per block
     const float *w_row;                    // gate/up with kPfScaleH: the plan's routing weight of every row
     float *out32;                          // down with kPfY32: y [Rp, R] in f32
@@ -66,7 +70,7 @@ struct PfArgs {
 // A task of the launch's last, partial round is split along K into pieces (at most kPfMaxPieces, whole super tiles
 // each); a piece stores its accumulators here (kPfPartBytes per workgroup).
 constexpr int kPfMaxPieces = 4;
-constexpr int kPfPartBytes = kPfWaves * kPfRtw * kPfTT * 64 * 16;
+constexpr int kPfPartBytes = kPfBWaves * kPfBRtw * kPfTT * 64 * 16;
 
 // Rounding forms of the epilogues (FORM, a compile-time set; the ragged kernels use none):
 constexpr int kPfRoundGU = 1;   // gate/up: g and u rounded to bf16 before the SwiGLU (the XLA einsums' bf16 outputs)
@@ -147,15 +151,17 @@ __device__ __forceinline__ void pf_ctile(const Cb3Wave &w, PfRegs &s, int st, co
     pf_steps<NTT, C, 0>(wv, cbrow, s.cbr, xrow, acc);
 }
 
+// Bytes per staged activation row of a 128-column tile (the block formats).  16-byte chunk c of row i sits at chunk
+// c ^ (i & 15): the 16 rows of an operand read, and the 16 chunks of a row written, fall on different banks.  A lane's
+// chunk of step j is act_chunk(q) plus a constant of j on other bits, so an exclusive or with that constant finds it.
+constexpr int kPfXRow = 256;
+
+template <class WP>
 struct PfShared {
-    union {
-        uint4 cbl[kPfWaves * 5 * 64];            // CB3: per-wavefront codebook slots (20 KB)
-        uint2 iq3grid[512];                      // IQ3_S: grid entry -> its 4 levels as f16 (4 KB)
-        uint32_t iq4pair[256];                   // IQ4_XS: byte -> f16 levels of its low and its high nibble (1 KB)
-        uint2 iq2code[1024];                     // IQ2_S: grid entry -> its 8 levels as codes 0..2, one byte each (8 KB)
-    };
-    uint32_t xs[2][kPfTm * kPfXPitch];           // column tiles ct (even/odd) of the block's rows, double-buffered;
-                                                 // gate/up epilogue: the gate accumulators of one (gate, up) pair
+    typename WP::Table tab;                      // the format's table, or CB3's codebook slots
+    // column tiles ct (even/odd) of the block's rows, double-buffered; gate/up epilogue: gate accumulators
+    static constexpr int kXBuf = kPfTm * (WP::kCols == 128 ? kPfXRow / 4 : kPfXPitch);
+    uint32_t xs[2][kXBuf];
     uint32_t xrowoff[kPfTm];                     // byte offset of every row's activations, or kXOut
     int last;                                    // split task: this workgroup's piece arrived last
 };
@@ -181,14 +187,18 @@ struct PfShared {
 
 // CB3: 160-column tiles of the code-tile layout; codebook slots per 640-column super tile (cb3_tiles.h).
 struct PfCb3 {
+    struct Table {
+        uint4 cbl[kPfWaves * 5 * 64];            // per-wavefront codebook slots (20 KB)
+    };
     static constexpr bool kLdsOnlyBarrier = false;
     static constexpr int kCols = kCb3TileCols;
     static constexpr bool kSplit = false;   // whole tasks only: K pieces measured slower (561 against 536 us)
+    static constexpr int kRtw = kPfRtw, kWaves = kPfWaves;
     static constexpr int kQOff = 4;
     using Wave = Cb3Wave;
     using Regs = PfRegs;
     static __device__ __forceinline__ int n_tiles(const PfArgs &a, int mat) { return (mat ? a.t1 : a.t0).CT; }
-    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, PfShared &sh, int mat, int e,
+    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, Table &sh, int mat, int e,
                                                 int rg, int wave, int lane, int st0, int st1) {
         const Cb3Table &tb = mat ? a.t1 : a.t0;
         const uint32_t *qt = tb.qs + (size_t)e * tb.CT * tb.RT * 256;
@@ -222,6 +232,61 @@ struct PfCb3 {
         pf_ctile<NTT, C>(w, s, st, xt, acc);
     }
 };
+
+// One column tile of a block format, software-pipelined over its 8 A operands f = 2 j + r (k-step j, row tile r): while
+// operand f meets the token tiles on the matrix cores, operand f + 1 is decoded and the table gathers of f + 2 are in
+// flight, one matrix-core instruction between every few vector ones.  The pipeline runs on across tiles (s.A: the next
+// tile's operand 0, s.g: the gathers of its operand 1), and each k-step's activations are read under the last row
+// tile's matrix-core work of the step before.
+//
+// Free of this order the compiler clumped a step's decode and its MFMAs and waited for each gather where it was
+// issued.
+template <class WP, int NTT, int C>
+__device__ __forceinline__ void pf_tile(const typename WP::Wave &w, typename WP::Regs &s, int st, const char *xb, uint32_t xoff,
+                                        f32x4 (&acc)[kPfBRtw][NTT]) {
+    constexpr int F = 4 * kPfBRtw;
+    const int ct = 4 * st + C;
+    uint4 b[NTT];
+#pragma unroll
+    for (int t = 0; t < NTT; ++t) b[t] = WP::acts(xb, xoff, t, 0);
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        const int r = f % kPfBRtw, j = f / kPfBRtw;
+        const int f1 = (f + 1) % F, f2 = (f + 2) % F;
+        const int c1 = f + 1 < F ? C : (C + 1) & 3, c2 = f + 2 < F ? C : (C + 1) & 3;
+        __builtin_amdgcn_sched_barrier(0);
+        const typename WP::Gather g2 = WP::gather(w, s.v[c2 & 1][f2 % kPfBRtw], c2, f2 / kPfBRtw);
+        const bf16x8 An = WP::weights8(w, s, c1, f1 % kPfBRtw, f1 / kPfBRtw);
+        if (f == F - 1) {
+            // this tile's plane words have all been decoded: their slot's next column tile (zeros past the range)
+#pragma unroll
+            for (int rr = 0; rr < kPfBRtw; ++rr) WP::load(w, ct + 2, s.v[C & 1][rr], rr, ct + 2 < w.CT);
+        }
+#pragma unroll
+        for (int t = 0; t < NTT; ++t) {
+            acc[r][t] = mfma16(s.A, b[t], acc[r][t]);
+            if (r == kPfBRtw - 1 && j < 3) b[t] = WP::acts(xb, xoff, t, j + 1);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x2, 6, 0);                       // the gathers' addresses
+        __builtin_amdgcn_sched_group_barrier(0x100, WP::kGathers, 0);
+#pragma unroll
+        for (int t = 0; t < NTT; ++t) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            if (r == kPfBRtw - 1 && j < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, (WP::kValu - 6 + NTT - 1) / NTT, 0);
+        }
+        s.A = An;
+        s.g = g2;
+    }
+}
+
+// The first operand of a row's first column tile (plane words in slot 0).
+template <class WP>
+__device__ __forceinline__ void pf_tile_begin(const typename WP::Wave &w, typename WP::Regs &s) {
+    s.g = WP::gather(w, s.v[0][0], 0, 0);
+    s.A = WP::weights8(w, s, 0, 0, 0);
+    s.g = WP::gather(w, s.v[0][1], 0, 0);
+}
 
 // IQ3_S: the reference's planes (planes.py:136-170, row on the minor axis) decoded straight into the matrix cores'
 // A operand.  A column tile is 128 columns = 8 words = half a 256-weight block.  In k-steps 2m and 2m + 1 (m = 0, 1)
@@ -271,14 +336,19 @@ struct PfIq3Wave {
 };
 struct PfIq3Regs {
     // plane words of column tile ct in slot ct & 1, per row tile: qs of words q and 4 + q, their sg words, qh, sc, d
-    uint32_t v[2][kPfRtw][7];
+    uint32_t v[2][kPfBRtw][7];
+    struct { uint2 lo, hi; } g;     // pf_tile's state: the next operand's gathers (levels of weights 0..3, 4..7) ...
+    bf16x8 A;                       // ... and the operand to multiply
 };
 
 struct PfIq3 {
+    struct Table {
+        uint2 iq3grid[512];                      // grid entry -> its 4 levels as f16 (4 KB)
+    };
     static constexpr bool kLdsOnlyBarrier = true;
     static constexpr bool kSplit = true;    // the last round's tasks split into K pieces
     static constexpr int kCols = kIq3TileCols;
-    static constexpr int kQOff = 8;
+    static constexpr int kRtw = kPfBRtw, kWaves = kPfBWaves;
     using Wave = PfIq3Wave;
     using Regs = PfIq3Regs;
     static __device__ __forceinline__ int n_tiles(const PfArgs &a, int mat) {
@@ -295,7 +365,7 @@ struct PfIq3 {
         u[5] = pf_word(w.sc + (size_t)(ct >> 1) * P, o, use);
         u[6] = pf_word(w.dd + (size_t)(ct >> 2) * P, o, use);
     }
-    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, PfShared &sh, int mat, int e,
+    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, Table &sh, int mat, int e,
                                                 int rg, int wave, int lane, int st0, int st1) {
         const Iq3Table &tb = mat ? a.i1 : a.i0;
         const size_t R = (size_t)tb.R;
@@ -306,28 +376,40 @@ struct PfIq3 {
         w.dd = (const char *)(tb.d + (size_t)e * ((tb.nblk + 1) / 2) * R);
         w.rpitch = 4u * (uint32_t)tb.R;
         w.q = lane >> 4;
-        w.lrow = 4u * (uint32_t)(rg * 64 + (lane & 15));
+        w.lrow = 4u * (uint32_t)(rg * 16 * kPfBRtw + (lane & 15));
         w.CT = min(tb.K / kIq3TileCols, 4 * st1);          // prefetch no column tile past the range
         w.grid = sh.iq3grid;
         (void)wave;
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int r = 0; r < kPfRtw; ++r) load(w, 4 * st0 + c, s.v[c][r], r, true);
+            for (int r = 0; r < kPfBRtw; ++r) load(w, 4 * st0 + c, s.v[c][r], r, true);
     }
-    // the 8 weights of step j of column tile ct for the row tile whose plane words are u
-    static __device__ __forceinline__ bf16x8 weights8(const Wave &w, const uint32_t (&u)[7], int ct, int j) {
+    static constexpr bool kHalfChunk = false;
+    static constexpr int kValu = 32, kGathers = 2;
+    using Gather = decltype(Regs::g);
+    static __device__ __forceinline__ uint32_t act_chunk(int q) { return 2 * q; }
+    static __device__ __forceinline__ uint4 acts(const char *xb, uint32_t xoff, int t, int j) {
+        return *(const uint4 *)(xb + t * 16 * kPfXRow + (xoff ^ 16 * (8 * (j >> 1) + (j & 1))));
+    }
+    // the grid entries of step j's 8 weights, column tile c (mod 4), for the row tile whose plane words are u
+    static __device__ __forceinline__ Gather gather(const Wave &w, const uint32_t (&u)[7], int, int j) {
+        const int m = j >> 1, half = j & 1;
+        const uint32_t word = m ? u[1] : u[0], qh4 = u[4] >> (4 * w.q) >> (16 * m);
+        const uint32_t i0 = ((word >> (16 * half)) & 255u) | (((qh4 >> (2 * half)) & 1u) << 8);
+        const uint32_t i1 = ((word >> (16 * half + 8)) & 255u) | (((qh4 >> (2 * half + 1)) & 1u) << 8);
+        return {w.grid[i0], w.grid[i1]};
+    }
+    // the 8 weights of step j of column tile c (mod 4), row tile r, from the gathers in s.g
+    static __device__ __forceinline__ bf16x8 weights8(const Wave &w, const Regs &s, int c, int r, int j) {
+        const uint32_t (&u)[7] = s.v[c & 1][r];
         const int m = j >> 1, half = j & 1, q = w.q;
-        const uint32_t word = m ? u[1] : u[0];
         // the word's 16 signs; sg2 has sign 2p at bit 2p and sign 2p + 1 at bit 2p + 16, a pair's two bf16 sign
         // bits once shifted left by 15 - 2p
         const uint32_t sg = ((m ? u[3] : u[2]) >> (16 * (q & 1))) & 0xffffu, sg2 = (sg << 15) | sg;
-        const uint32_t qh4 = u[4] >> (4 * q) >> (16 * m);
-        const uint32_t nib = (u[5] >> (4 * (q >> 1)) >> (16 * (ct & 1) + 8 * m)) & 15u;
-        const float scale = f16_bits_to_f32(u[6] >> (16 * ((ct >> 1) & 1))) * (float)(1u + 2u * nib);
-        const uint32_t i0 = ((word >> (16 * half)) & 255u) | (((qh4 >> (2 * half)) & 1u) << 8);
-        const uint32_t i1 = ((word >> (16 * half + 8)) & 255u) | (((qh4 >> (2 * half + 1)) & 1u) << 8);
-        const uint2 g0 = w.grid[i0], g1 = w.grid[i1];
+        const uint32_t nib = (u[5] >> (4 * (q >> 1)) >> (16 * (c & 1) + 8 * m)) & 15u;
+        const float scale = f16_bits_to_f32(u[6] >> (16 * (c >> 1))) * (float)(1u + 2u * nib);
+        const uint2 g0 = s.g.lo, g1 = s.g.hi;
         const int sh = 15 - 8 * half;
         uint4 A;
         A.x = pf_bf16_pair(pf_mix<0>(g0.x, scale), pf_mix<1>(g0.x, scale)) ^ ((sg2 << sh) & 0x80008000u);
@@ -337,29 +419,9 @@ struct PfIq3 {
         return __builtin_bit_cast(bf16x8, A);
     }
     template <int NTT, int C>
-    static __device__ __forceinline__ void tile(const Wave &w, Regs &s, int st, const uint32_t *xt,
-                                                f32x4 (&acc)[kPfRtw][NTT]) {
-        const int ct = 4 * st + C;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (j > 0) __builtin_amdgcn_sched_barrier(0);
-            uint4 b[NTT];
-#pragma unroll
-            for (int tt = 0; tt < NTT; ++tt)
-                b[tt] = *(const uint4 *)(xt + tt * 16 * kPfXPitch + 32 * (j >> 1) + 4 * (j & 1));
-            bf16x8 A = weights8(w, s.v[C & 1][0], ct, j);
-#pragma unroll
-            for (int r = 0; r < kPfRtw; ++r) {
-                bf16x8 An = A;
-                if (r + 1 < kPfRtw) An = weights8(w, s.v[C & 1][r + 1], ct, j);
-#pragma unroll
-                for (int tt = 0; tt < NTT; ++tt) acc[r][tt] = mfma16(A, b[tt], acc[r][tt]);
-                A = An;
-            }
-        }
-        // the slot's next column tile (ct + 2); past the row's end the loads read zeros (the slot is not read again)
-#pragma unroll
-        for (int r = 0; r < kPfRtw; ++r) load(w, ct + 2, s.v[C & 1][r], r, ct + 2 < w.CT);
+    static __device__ __forceinline__ void tile(const Wave &w, Regs &s, int st, const char *xb, uint32_t xoff,
+                                                f32x4 (&acc)[kPfBRtw][NTT]) {
+        pf_tile<PfIq3, NTT, C>(w, s, st, xb, xoff, acc);
     }
 };
 
@@ -377,14 +439,24 @@ struct PfIq2Wave {
     const uint2 *code;                      // LDS: grid entry -> 8 level codes
 };
 struct PfIq2Regs {
-    uint32_t v[2][kPfRtw][5];   // column tile ct in slot ct & 1, per row tile: the lane's qs and sg words, qh, sc, d
+    uint32_t v[2][kPfBRtw][5];   // column tile ct in slot ct & 1, per row tile: the lane's qs and sg words, qh, sc, d
+    // The scaled levels of one 16-weight scale group as a byte table: entry c (0..2) is bf16(level c * scale), entry
+    // c + 4 its negative; low bytes, high bytes, high bytes of the negatives.
+    struct Levels {
+        uint32_t lo, hi, neg;
+    } lv[kPfBRtw];               // per row tile, steps 2 jj and 2 jj + 1
+    uint2 g;                    // pf_tile's state: the next operand's gather (8 level codes) ...
+    bf16x8 A;                   // ... and the operand to multiply
 };
 
 struct PfIq2 {
+    struct Table {
+        uint2 iq2code[1024];                     // grid entry -> its 8 levels as codes 0..2, one byte each (8 KB)
+    };
     static constexpr bool kLdsOnlyBarrier = true;
     static constexpr bool kSplit = true;    // the last round's tasks split into K pieces
     static constexpr int kCols = 128;
-    static constexpr int kQOff = 16;       // dwords: word q of the tile
+    static constexpr int kRtw = kPfBRtw, kWaves = kPfBWaves;
     using Wave = PfIq2Wave;
     using Regs = PfIq2Regs;
     static __device__ __forceinline__ int n_tiles(const PfArgs &a, int mat) { return (mat ? a.j1 : a.j0).K / 128; }
@@ -396,7 +468,7 @@ struct PfIq2 {
         u[3] = pf_word(w.sc + (size_t)ct * P, o, use);
         u[4] = pf_word(w.dd + (size_t)(ct >> 2) * P, o, use);
     }
-    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, PfShared &sh, int mat, int e,
+    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, Table &sh, int mat, int e,
                                                 int rg, int wave, int lane, int st0, int st1) {
         const Iq2Table &tb = mat ? a.j1 : a.j0;
         const size_t R = (size_t)tb.R;
@@ -407,68 +479,51 @@ struct PfIq2 {
         w.dd = (const char *)(tb.d + (size_t)e * ((tb.nblk + 1) / 2) * R);
         w.rpitch = 4u * (uint32_t)tb.R;
         w.q = lane >> 4;
-        w.lrow = 4u * (uint32_t)(rg * 64 + (lane & 15));
+        w.lrow = 4u * (uint32_t)(rg * 16 * kPfBRtw + (lane & 15));
         w.CT = min(tb.K / 128, 4 * st1);                   // prefetch no column tile past the range
         w.code = sh.iq2code;
         (void)wave;
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int r = 0; r < kPfRtw; ++r) load(w, 4 * st0 + c, s.v[c][r], r, true);
+            for (int r = 0; r < kPfBRtw; ++r) load(w, 4 * st0 + c, s.v[c][r], r, true);
     }
-    // The scaled levels of one 16-weight scale group as a byte table: entry c (0..2) is bf16(level c * scale), entry
-    // c + 4 its negative; low bytes, high bytes, high bytes of the negatives.
-    struct Levels {
-        uint32_t lo, hi, neg;
-    };
-    static __device__ __forceinline__ Levels levels(const Wave &w, const uint32_t (&u)[5], int ct, int jj) {
+    static constexpr bool kHalfChunk = false;
+    static constexpr int kValu = 26, kGathers = 1;
+    using Gather = uint2;
+    static __device__ __forceinline__ uint32_t act_chunk(int q) { return 4 * q; }
+    static __device__ __forceinline__ uint4 acts(const char *xb, uint32_t xoff, int t, int j) {
+        return *(const uint4 *)(xb + t * 16 * kPfXRow + (xoff ^ 16 * j));
+    }
+    static __device__ __forceinline__ PfIq2Regs::Levels levels(const Wave &w, const uint32_t (&u)[5], int c, int jj) {
         const uint32_t nib = (u[3] >> (8 * w.q) >> (4 * jj)) & 15u;
-        const float scale = f16_bits_to_f32(u[4] >> (16 * ((ct >> 1) & 1))) * 0.25f * (0.5f + (float)nib);
+        const float scale = f16_bits_to_f32(u[4] >> (16 * (c >> 1))) * 0.25f * (0.5f + (float)nib);
         const uint32_t c01 = pf_bf16_pair(8.0f * scale, 25.0f * scale), c2 = pf_bf16_pair(43.0f * scale, 0.0f);
-        Levels t;
+        PfIq2Regs::Levels t;
         t.lo = perm(c2, c01, 0x0c040200u);
         t.hi = perm(c2, c01, 0x0c050301u);
         t.neg = t.hi ^ 0x80808080u;
         return t;
     }
-    // the 8 weights of step j (group j of the lane's word) for the row tile whose plane words are u
-    static __device__ __forceinline__ bf16x8 weights8(const Wave &w, const uint32_t (&u)[5], const Levels &t, int j) {
-        const uint32_t idx = ((u[0] >> (8 * j)) & 255u) | (((u[2] >> (8 * w.q) >> (2 * j)) & 3u) << 8);
-        const uint2 c = w.code[idx];
+    // the level codes of step j (group j of the lane's word) for the row tile whose plane words are u
+    static __device__ __forceinline__ Gather gather(const Wave &w, const uint32_t (&u)[5], int, int j) {
+        return w.code[((u[0] >> (8 * j)) & 255u) | (((u[2] >> (8 * w.q) >> (2 * j)) & 3u) << 8)];
+    }
+    // the 8 weights of step j of column tile c (mod 4), row tile r, from the gather in s.g
+    static __device__ __forceinline__ bf16x8 weights8(const Wave &w, Regs &s, int c, int r, int j) {
+        const uint32_t (&u)[5] = s.v[c & 1][r];
+        if ((j & 1) == 0) s.lv[r] = levels(w, u, c, j >> 1);
+        const PfIq2Regs::Levels &t = s.lv[r];
         // 4 sign bits to bit 2 of 4 bytes: one 24-bit multiply (shifts by 2, 9, 16, 23: no two bits meet)
         const uint32_t s0 = __umul24((u[1] >> (8 * j)) & 15u, 0x810204u) & 0x04040404u;
         const uint32_t s1 = __umul24((u[1] >> (8 * j + 4)) & 15u, 0x810204u) & 0x04040404u;
-        const uint2 a0 = pf_lookup4(t.lo, t.lo, t.hi, t.neg, c.x | s0), a1 = pf_lookup4(t.lo, t.lo, t.hi, t.neg, c.y | s1);
+        const uint2 a0 = pf_lookup4(t.lo, t.lo, t.hi, t.neg, s.g.x | s0), a1 = pf_lookup4(t.lo, t.lo, t.hi, t.neg, s.g.y | s1);
         return __builtin_bit_cast(bf16x8, make_uint4(a0.x, a0.y, a1.x, a1.y));
     }
     template <int NTT, int C>
-    static __device__ __forceinline__ void tile(const Wave &w, Regs &s, int st, const uint32_t *xt,
-                                                f32x4 (&acc)[kPfRtw][NTT]) {
-        const int ct = 4 * st + C;
-        Levels lv[kPfRtw];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (j > 0) __builtin_amdgcn_sched_barrier(0);
-            uint4 b[NTT];
-#pragma unroll
-            for (int tt = 0; tt < NTT; ++tt) b[tt] = *(const uint4 *)(xt + tt * 16 * kPfXPitch + 4 * j);
-            if ((j & 1) == 0) lv[0] = levels(w, s.v[C & 1][0], ct, j >> 1);
-            bf16x8 A = weights8(w, s.v[C & 1][0], lv[0], j);
-#pragma unroll
-            for (int r = 0; r < kPfRtw; ++r) {
-                bf16x8 An = A;
-                if (r + 1 < kPfRtw) {
-                    if ((j & 1) == 0) lv[r + 1] = levels(w, s.v[C & 1][r + 1], ct, j >> 1);
-                    An = weights8(w, s.v[C & 1][r + 1], lv[r + 1], j);
-                }
-#pragma unroll
-                for (int tt = 0; tt < NTT; ++tt) acc[r][tt] = mfma16(A, b[tt], acc[r][tt]);
-                A = An;
-            }
-        }
-        // the slot's next column tile (ct + 2); past the row's end the loads read zeros (the slot is not read again)
-#pragma unroll
-        for (int r = 0; r < kPfRtw; ++r) load(w, ct + 2, s.v[C & 1][r], r, ct + 2 < w.CT);
+    static __device__ __forceinline__ void tile(const Wave &w, Regs &s, int st, const char *xb, uint32_t xoff,
+                                                f32x4 (&acc)[kPfBRtw][NTT]) {
+        pf_tile<PfIq2, NTT, C>(w, s, st, xb, xoff, acc);
     }
 };
 
@@ -485,15 +540,18 @@ struct PfKqWave {
     int q, CT;
 };
 struct PfKqRegs {
-    uint32_t v[2][kPfRtw][7];   // column tile ct in slot ct & 1, per row tile: qs words 2q, 2q + 1, sc x 2, d, hm x 2
+    uint32_t v[2][kPfBRtw][7];   // column tile ct in slot ct & 1, per row tile: qs words 2q, 2q + 1, sc x 2, d, hm x 2
+    struct {} g;                // pf_tile's state: no gathers, the operand to multiply
+    bf16x8 A;
 };
 
 template <bool Q3>
 struct PfKq {
+    struct Table {};
     static constexpr bool kLdsOnlyBarrier = true;
     static constexpr bool kSplit = true;    // the last round's tasks split into K pieces
     static constexpr int kCols = 128;
-    static constexpr int kQOff = 4;        // dwords: columns 8q .. 8q+7 of a 32-column stripe
+    static constexpr int kRtw = kPfBRtw, kWaves = kPfBWaves;
     using Wave = PfKqWave;
     using Regs = PfKqRegs;
     static __device__ __forceinline__ int n_tiles(const PfArgs &a, int mat) { return (mat ? a.q1 : a.q0).K / 128; }
@@ -511,7 +569,7 @@ struct PfKq {
             u[6] = pf_word(w.hm + (size_t)(8 * b) * P, ob, use);
         }
     }
-    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, PfShared &sh, int mat, int e,
+    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, Table &sh, int mat, int e,
                                                 int rg, int wave, int lane, int st0, int st1) {
         const KqTable &tb = mat ? a.q1 : a.q0;
         const size_t R = (size_t)tb.R;
@@ -521,14 +579,14 @@ struct PfKq {
         w.hm = Q3 ? (const char *)(tb.hm + (size_t)e * 8 * tb.nblk * R) : nullptr;
         w.rpitch = 4u * (uint32_t)tb.R;
         w.q = lane >> 4;
-        w.lrow = 4u * (uint32_t)(rg * 64 + (lane & 15));
+        w.lrow = 4u * (uint32_t)(rg * 16 * kPfBRtw + (lane & 15));
         w.CT = min(tb.K / 128, 4 * st1);                   // prefetch no column tile past the range
         (void)sh;
         (void)wave;
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int r = 0; r < kPfRtw; ++r) load(w, 4 * st0 + c, s.v[c][r], r, true);
+            for (int r = 0; r < kPfBRtw; ++r) load(w, 4 * st0 + c, s.v[c][r], r, true);
     }
     // 4 weights from the 4 byte-sized values of t (each 0..3, Q3_K 0..7): f32 -> bf16 pairs
     static __device__ __forceinline__ uint2 four(uint32_t t, float m, float a) {
@@ -536,9 +594,18 @@ struct PfKq {
         const float v2 = (float)((t >> 16) & 255u), v3 = (float)(t >> 24);
         return make_uint2(pf_bf16_pair(fmaf(v0, m, a), fmaf(v1, m, a)), pf_bf16_pair(fmaf(v2, m, a), fmaf(v3, m, a)));
     }
-    // the 8 weights of step j (shift stripe j) for the row tile whose plane words are u
-    static __device__ __forceinline__ bf16x8 weights8(const Wave &w, const uint32_t (&u)[7], int ct, int j) {
-        const int n = ct & 1;
+    static constexpr bool kHalfChunk = false;
+    static constexpr int kValu = Q3 ? 34 : 27, kGathers = 0;
+    using Gather = decltype(Regs::g);
+    static __device__ __forceinline__ uint32_t act_chunk(int q) { return q; }
+    static __device__ __forceinline__ uint4 acts(const char *xb, uint32_t xoff, int t, int j) {
+        return *(const uint4 *)(xb + t * 16 * kPfXRow + (xoff ^ 16 * (4 * j)));
+    }
+    static __device__ __forceinline__ Gather gather(const Wave &, const uint32_t (&)[7], int, int) { return {}; }
+    // the 8 weights of step j (shift stripe j) of column tile c (mod 4), row tile r
+    static __device__ __forceinline__ bf16x8 weights8(const Wave &w, const Regs &s, int c, int r, int j) {
+        const uint32_t (&u)[7] = s.v[c & 1][r];
+        const int n = c & 1;
         const uint32_t sb = ((j >> 1 ? u[3] : u[2]) >> (16 * (j & 1) + 8 * (w.q >> 1))) & 255u;
         const float d = f16_bits_to_f32(u[4] & 0xffffu);
         uint32_t t0 = (u[0] >> (2 * j)) & 0x03030303u, t1 = (u[1] >> (2 * j)) & 0x03030303u;
@@ -561,28 +628,9 @@ struct PfKq {
         return __builtin_bit_cast(bf16x8, make_uint4(l0.x, l0.y, l1.x, l1.y));
     }
     template <int NTT, int C>
-    static __device__ __forceinline__ void tile(const Wave &w, Regs &s, int st, const uint32_t *xt,
-                                                f32x4 (&acc)[kPfRtw][NTT]) {
-        const int ct = 4 * st + C;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (j > 0) __builtin_amdgcn_sched_barrier(0);
-            uint4 b[NTT];
-#pragma unroll
-            for (int tt = 0; tt < NTT; ++tt) b[tt] = *(const uint4 *)(xt + tt * 16 * kPfXPitch + 16 * j);
-            bf16x8 A = weights8(w, s.v[C & 1][0], ct, j);
-#pragma unroll
-            for (int r = 0; r < kPfRtw; ++r) {
-                bf16x8 An = A;
-                if (r + 1 < kPfRtw) An = weights8(w, s.v[C & 1][r + 1], ct, j);
-#pragma unroll
-                for (int tt = 0; tt < NTT; ++tt) acc[r][tt] = mfma16(A, b[tt], acc[r][tt]);
-                A = An;
-            }
-        }
-        // the slot's next column tile (ct + 2); past the row's end the loads read zeros (the slot is not read again)
-#pragma unroll
-        for (int r = 0; r < kPfRtw; ++r) load(w, ct + 2, s.v[C & 1][r], r, ct + 2 < w.CT);
+    static __device__ __forceinline__ void tile(const Wave &w, Regs &s, int st, const char *xb, uint32_t xoff,
+                                                f32x4 (&acc)[kPfBRtw][NTT]) {
+        pf_tile<PfKq<Q3>, NTT, C>(w, s, st, xb, xoff, acc);
     }
 };
 
@@ -600,14 +648,19 @@ struct PfIq4Wave {
     const uint32_t *pair;                   // LDS: byte -> its two levels as f16
 };
 struct PfIq4Regs {
-    uint32_t v[2][kPfRtw][7];   // column tile ct in slot ct & 1, per row tile: the 4 words, sl, sh, d
+    uint32_t v[2][kPfBRtw][7];   // column tile ct in slot ct & 1, per row tile: the 4 words, sl, sh, d
+    uint4 g;                    // pf_tile's state: the next operand's gathers (level pairs of the word's 4 bytes) ...
+    bf16x8 A;                   // ... and the operand to multiply
 };
 
 struct PfIq4 {
+    struct Table {
+        uint32_t iq4pair[256];                   // byte -> f16 levels of its low and its high nibble (1 KB)
+    };
     static constexpr bool kLdsOnlyBarrier = true;
     static constexpr bool kSplit = true;    // the last round's tasks split into K pieces
     static constexpr int kCols = 128;
-    static constexpr int kQOff = 2;        // dwords: columns 4q .. 4q+3 of a 32-column group
+    static constexpr int kRtw = kPfBRtw, kWaves = kPfBWaves;
     using Wave = PfIq4Wave;
     using Regs = PfIq4Regs;
     static __device__ __forceinline__ int n_tiles(const PfArgs &a, int mat) { return (mat ? a.k1 : a.k0).K / 128; }
@@ -619,7 +672,7 @@ struct PfIq4 {
         u[5] = pf_word(w.sh + (size_t)(ct >> 1) * P, o, use);
         u[6] = pf_word(w.dd + (size_t)(ct >> 2) * P, o, use);
     }
-    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, PfShared &sh, int mat, int e,
+    static __device__ __forceinline__ void init(Wave &w, Regs &s, const PfArgs &a, Table &sh, int mat, int e,
                                                 int rg, int wave, int lane, int st0, int st1) {
         const Iq4Table &tb = mat ? a.k1 : a.k0;
         const size_t R = (size_t)tb.R;
@@ -629,57 +682,49 @@ struct PfIq4 {
         w.dd = (const char *)(tb.d + (size_t)e * ((tb.nblk + 1) / 2) * R);
         w.rpitch = 4u * (uint32_t)tb.R;
         w.q = lane >> 4;
-        w.lrow = 4u * (uint32_t)(rg * 64 + (lane & 15));
+        w.lrow = 4u * (uint32_t)(rg * 16 * kPfBRtw + (lane & 15));
         w.CT = min(tb.K / 128, 4 * st1);                   // prefetch no column tile past the range
         w.pair = sh.iq4pair;
         (void)wave;
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int r = 0; r < kPfRtw; ++r) load(w, 4 * st0 + c, s.v[c][r], r, true);
+            for (int r = 0; r < kPfBRtw; ++r) load(w, 4 * st0 + c, s.v[c][r], r, true);
     }
-    // the 8 weights of step j (sub-block 4 (ct % 2) + j) for the row tile whose plane words are u
-    static __device__ __forceinline__ bf16x8 weights8(const Wave &w, const uint32_t (&u)[7], int ct, int j) {
-        const int i = 4 * (ct & 1) + j;
-        const int sv = (int)(((u[4] >> (4 * i)) & 15u) | (((u[5] >> (2 * i)) & 3u) << 4)) - 32;
-        const float scale = f16_bits_to_f32(u[6] >> (16 * ((ct >> 1) & 1))) * (float)sv;
+    static constexpr bool kHalfChunk = true;
+    static constexpr int kValu = 24, kGathers = 4;
+    using Gather = uint4;
+    static __device__ __forceinline__ uint32_t act_chunk(int q) { return q >> 1; }      // odd lane groups: its second half
+    static __device__ __forceinline__ uint4 acts(const char *xb, uint32_t xoff, int t, int j) {
+        const char *row = xb + t * 16 * kPfXRow;
+        const uint2 lo = *(const uint2 *)(row + (xoff ^ 16 * (4 * j)));
+        const uint2 hi = *(const uint2 *)(row + (xoff ^ 16 * (4 * j + 2)));
+        return make_uint4(lo.x, lo.y, hi.x, hi.y);
+    }
+    // the level pairs of step j's word for the row tile whose plane words are u (one read per nibble from 16 entries,
+    // free of bank conflicts, costs more in extra instructions than the conflicts do: down 128 -> 151 us at 27 tokens)
+    static __device__ __forceinline__ Gather gather(const Wave &w, const uint32_t (&u)[7], int, int j) {
         const uint32_t x = u[j];
-        const uint32_t p0 = w.pair[x & 255u], p1 = w.pair[(x >> 8) & 255u], p2 = w.pair[(x >> 16) & 255u],
-                       p3 = w.pair[x >> 24];
+        return make_uint4(w.pair[x & 255u], w.pair[(x >> 8) & 255u], w.pair[(x >> 16) & 255u], w.pair[x >> 24]);
+    }
+    // the 8 weights of step j (sub-block 4 (c % 2) + j) of column tile c (mod 4), row tile r, from the gathers in s.g
+    static __device__ __forceinline__ bf16x8 weights8(const Wave &, const Regs &s, int c, int r, int j) {
+        const uint32_t (&u)[7] = s.v[c & 1][r];
+        const int i = 4 * (c & 1) + j;
+        const int sv = (int)(((u[4] >> (4 * i)) & 15u) | (((u[5] >> (2 * i)) & 3u) << 4)) - 32;
+        const float scale = f16_bits_to_f32(u[6] >> (16 * (c >> 1))) * (float)sv;
+        const uint4 p = s.g;
         uint4 A;
-        A.x = pf_bf16_pair(pf_mix<0>(p0, scale), pf_mix<0>(p1, scale));
-        A.y = pf_bf16_pair(pf_mix<0>(p2, scale), pf_mix<0>(p3, scale));
-        A.z = pf_bf16_pair(pf_mix<1>(p0, scale), pf_mix<1>(p1, scale));
-        A.w = pf_bf16_pair(pf_mix<1>(p2, scale), pf_mix<1>(p3, scale));
+        A.x = pf_bf16_pair(pf_mix<0>(p.x, scale), pf_mix<0>(p.y, scale));
+        A.y = pf_bf16_pair(pf_mix<0>(p.z, scale), pf_mix<0>(p.w, scale));
+        A.z = pf_bf16_pair(pf_mix<1>(p.x, scale), pf_mix<1>(p.y, scale));
+        A.w = pf_bf16_pair(pf_mix<1>(p.z, scale), pf_mix<1>(p.w, scale));
         return __builtin_bit_cast(bf16x8, A);
     }
     template <int NTT, int C>
-    static __device__ __forceinline__ void tile(const Wave &w, Regs &s, int st, const uint32_t *xt,
-                                                f32x4 (&acc)[kPfRtw][NTT]) {
-        const int ct = 4 * st + C;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (j > 0) __builtin_amdgcn_sched_barrier(0);
-            uint4 b[NTT];
-#pragma unroll
-            for (int tt = 0; tt < NTT; ++tt) {
-                const uint2 lo = *(const uint2 *)(xt + tt * 16 * kPfXPitch + 16 * j);
-                const uint2 hi = *(const uint2 *)(xt + tt * 16 * kPfXPitch + 16 * j + 8);
-                b[tt] = make_uint4(lo.x, lo.y, hi.x, hi.y);
-            }
-            bf16x8 A = weights8(w, s.v[C & 1][0], ct, j);
-#pragma unroll
-            for (int r = 0; r < kPfRtw; ++r) {
-                bf16x8 An = A;
-                if (r + 1 < kPfRtw) An = weights8(w, s.v[C & 1][r + 1], ct, j);
-#pragma unroll
-                for (int tt = 0; tt < NTT; ++tt) acc[r][tt] = mfma16(A, b[tt], acc[r][tt]);
-                A = An;
-            }
-        }
-        // the slot's next column tile (ct + 2); past the row's end the loads read zeros (the slot is not read again)
-#pragma unroll
-        for (int r = 0; r < kPfRtw; ++r) load(w, ct + 2, s.v[C & 1][r], r, ct + 2 < w.CT);
+    static __device__ __forceinline__ void tile(const Wave &w, Regs &s, int st, const char *xb, uint32_t xoff,
+                                                f32x4 (&acc)[kPfBRtw][NTT]) {
+        pf_tile<PfIq4, NTT, C>(w, s, st, xb, xoff, acc);
     }
 };
 
@@ -687,14 +732,17 @@ struct PfIq4 {
 // piece / np: the workgroup runs super tiles [piece n_st / np, (piece + 1) n_st / np) of the task (np == 1: all of
 // them); sti: the split task's index among the launch's split tasks (counter and piece sums).
 template <int MODE, int NTT, class WP, int FORM>
-__device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int g, int rbg, int e, int n, int piece,
+__device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP> &sh, int g, int rbg, int e, int n, int piece,
                                              int np, int sti) {
     uint32_t *xs = &sh.xs[0][0], *xrowoff = sh.xrowoff;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row0 = g * kPfTm;
     const int mat = MODE == 0 ? (wave & 1) : 0;
-    const int rg = rbg * a.wg_rows + (MODE == 0 ? (wave >> 1) : wave);   // 64-row group of this wavefront
+    constexpr int kRtw = WP::kRtw, kWaves = WP::kWaves;
+    constexpr bool kBlock = WP::kCols == 128;             // a block format
+    // this wavefront's group of 16 kRtw rows
+    const int rg = rbg * (kWaves >> (MODE == 0)) + (MODE == 0 ? (wave >> 1) : wave);
 
     const int CT = WP::n_tiles(a, mat);
     const int n_st = (CT + 3) >> 2;                     // super tiles of a row (the last one maybe partial)
@@ -702,15 +750,15 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int 
     const int ct_end = min(CT, 4 * s1);
     typename WP::Wave w;
     typename WP::Regs s;
-    WP::init(w, s, a, sh, mat, e, rg, wave, lane, s0, s1);
+    WP::init(w, s, a, sh.tab, mat, e, rg, wave, lane, s0, s1);
 
     // activation tile: the block's 16 NTT rows x kXU uint4 (WP::kCols columns), staged as buffer loads by
     // kXRows x kXU threads, kXRows rows per pass (thread t: row t / kXU + kXRows j, uint4 column t % kXU), so every
     // pass is a constant offset from the first; rows >= n and columns >= K take an offset past the buffer's range,
     // which reads zero
     constexpr int kXU = WP::kCols / 8;                        // 20 (CB3) or 16 (IQ3_S)
-    constexpr int kXRows = (64 * kPfWaves) / kXU;             // 12 or 16
-    constexpr int kXBuf = kPfTm * kPfXPitch;                  // dwords per tile buffer
+    constexpr int kXRows = (64 * kWaves) / kXU;               // 12 or 32
+    constexpr int kXBuf = PfShared<WP>::kXBuf;                // dwords per tile buffer
     constexpr int kXJ = (16 * NTT + kXRows - 1) / kXRows;
     const __amdgpu_buffer_rsrc_t xbuf =
         __builtin_amdgcn_make_buffer_rsrc((void *)a.x, (short)0, (int)a.x_bytes, kBufferWord3);
@@ -723,35 +771,47 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int 
     const int xr0 = tid / kXU, xc8 = tid - xr0 * kXU;
     const bool stager = tid < kXRows * kXU;
     uint4 xr[kXJ];
-    // use: whether the tile is staged at all (no branch around the loads: past the range they read zeros)
+    // byte offset of the thread's piece j in column tile 0; the block formats hold theirs in registers for the whole
+    // row (read from LDS at every tile they were a chain of LDS latencies at its start; CB3 has no registers left)
+    auto piece_off = [&](int j) {
+        const int row = xr0 + kXRows * j;
+        return stager && row < 16 * NTT ? xrowoff[row] + 16u * (uint32_t)xc8 : kXOut;
+    };
+    uint32_t xo[kXJ];
+    if constexpr (kBlock) {
+#pragma unroll
+        for (int j = 0; j < kXJ; ++j) xo[j] = piece_off(j);
+    }
+    const __amdgpu_buffer_rsrc_t xnull = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, (short)0, 0, kBufferWord3);
+    // use: whether the tile is staged at all (no branch around the loads: from an empty range they read zeros)
     auto load_x = [&](int ct, bool use) {
         const int lim = (a.K - WP::kCols * ct) >> 3;          // uint4 columns of this tile inside the row
+        const __amdgpu_buffer_rsrc_t r = use ? xbuf : xnull;
 #pragma unroll
         for (int j = 0; j < kXJ; ++j) {
-            const int row = xr0 + kXRows * j;
-            uint32_t o = kXOut;
-            if (use && stager && row < 16 * NTT && xc8 < lim)
-                o = xrowoff[row] + 16u * (uint32_t)xc8 + (uint32_t)(2 * WP::kCols * ct);
-            xr[j] = bload(xbuf, o, 0);
+            // K is whole 128-column tiles; a CB3 row may end inside its last 160-column tile
+            const uint32_t o = kBlock ? xo[j] : xc8 < lim ? piece_off(j) : kXOut;
+            xr[j] = bload(r, o, (uint32_t)(2 * WP::kCols * ct));
         }
     };
     auto store_x = [&](int buf) {
 #pragma unroll
         for (int j = 0; j < kXJ; ++j) {
             const int row = xr0 + kXRows * j;
-            if (stager && row < 16 * NTT) *(uint4 *)(xs + buf * kXBuf + row * kPfXPitch + 4 * xc8) = xr[j];
+            const int at = kBlock ? row * (kPfXRow / 4) + 4 * (xc8 ^ (row & 15)) : row * kPfXPitch + 4 * xc8;
+            if (stager && row < 16 * NTT) *(uint4 *)(xs + buf * kXBuf + at) = xr[j];
         }
     };
     load_x(4 * s0, true);
+    if constexpr (kBlock) pf_tile_begin<WP>(w, s);      // the format's LDS table: published above
     store_x(0);
 
-    f32x4 acc[kPfRtw][NTT];
+    f32x4 acc[kRtw][NTT];
 #pragma unroll
-    for (int r = 0; r < kPfRtw; ++r)
+    for (int r = 0; r < kRtw; ++r)
 #pragma unroll
         for (int t = 0; t < NTT; ++t) acc[r][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
     const int jt = lane & 15, q = lane >> 4;
-    const uint32_t *xrow = xs + jt * kPfXPitch + WP::kQOff * q;
 
     // one barrier per column tile: tile ct sits in buffer ct & 1 (= C & 1); the next tile's loads are issued first
     // (ahead of this tile's code and codebook loads, so waiting for them never waits for those) and stored into the
@@ -769,7 +829,10 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int 
             __syncthreads();
             if (ct + 1 < ct_end) load_x(ct + 1, true);
         }
-        WP::template tile<NTT, C>(w, s, st, xrow + (C & 1) * kXBuf, acc);
+        if constexpr (kBlock)
+            WP::template tile<NTT, C>(w, s, st, (const char *)(xs + (C & 1) * kXBuf),
+                                      jt * kPfXRow + 16 * (WP::act_chunk(q) ^ jt) + (WP::kHalfChunk ? 8 * (q & 1) : 0), acc);
+        else WP::template tile<NTT, C>(w, s, st, xs + jt * kPfXPitch + WP::kQOff * q + (C & 1) * kXBuf, acc);
         if (ct + 1 < ct_end) store_x((C + 1) & 1);
     };
     const int st_full = min(CT >> 2, s1);
@@ -793,14 +856,14 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int 
         const __amdgpu_buffer_rsrc_t pr =
             __builtin_amdgcn_make_buffer_rsrc((void *)a.part, (short)0, 0x7fffffff, kBufferWord3);
         const uint32_t lane_off = 16u * (uint32_t)lane;
-        auto piece_off = [&](int pc, int r, int t) {
+        auto part_off = [&](int pc, int r, int t) {
             return (uint32_t)(sti * np + pc) * (uint32_t)kPfPartBytes +
-                   (uint32_t)((wave * kPfRtw + r) * kPfTT + t) * 1024u + lane_off;
+                   (uint32_t)((wave * kRtw + r) * kPfTT + t) * 1024u + lane_off;
         };
 #pragma unroll
-        for (int r = 0; r < kPfRtw; ++r)
+        for (int r = 0; r < kRtw; ++r)
 #pragma unroll
-            for (int t = 0; t < NTT; ++t) wt_store4(pr, piece_off(piece, r, t), acc[r][t]);
+            for (int t = 0; t < NTT; ++t) wt_store4(pr, part_off(piece, r, t), acc[r][t]);
         __builtin_amdgcn_s_waitcnt(0);                  // this wavefront's stores have completed
         __syncthreads();                                // ... and every wavefront's
         if (tid == 0) sh.last = counter_add(a.cnt + sti, 1u) == (uint32_t)(np - 1);
@@ -809,34 +872,38 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int 
         if (tid == 0) counter_reset(a.cnt + sti);       // zero again for the next launch
         // every piece's sums from memory, this one's too (its stores have completed), added in piece order
 #pragma unroll
-        for (int r = 0; r < kPfRtw; ++r)
+        for (int r = 0; r < kRtw; ++r)
 #pragma unroll
             for (int t = 0; t < NTT; ++t) acc[r][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
         for (int pc = 0; pc < np; ++pc) {
 #pragma unroll
-            for (int r = 0; r < kPfRtw; ++r)
+            for (int r = 0; r < kRtw; ++r)
 #pragma unroll
                 for (int t = 0; t < NTT; ++t)
-                    acc[r][t] += coherent_load4(pr, piece_off(pc, r, t));
+                    acc[r][t] += coherent_load4(pr, part_off(pc, r, t));
         }
     }
 
     // epilogue: lane (jt, q) holds rows 16 r + 4 q + i (i = 0..3) of the wavefront's 64 rows for tokens 16 t + jt
-    const int rbase = rg * 64;
+    const int rbase = rg * 16 * kRtw;
     if constexpr (MODE == 0) {
-        float *gbuf = (float *)xs;                           // [64 rows][kPfGPitch] gate accumulators of one pair
-        for (int pair = 0; pair < 2; ++pair) {
+        // gate accumulators of as many (gate, up) pairs as the activation buffers hold at once: [rows][kPfGPitch]
+        constexpr int kPairs = kBlock ? kWaves / 2 : 1;
+        static_assert(kPairs * 16 * kRtw * kPfGPitch <= 2 * kXBuf, "the exchange fits the tile buffers");
+        float *gbuf = (float *)xs + (kPairs > 1 ? (wave >> 1) * 16 * kRtw * kPfGPitch : 0);
+        for (int pair = 0; pair < kWaves / 2; pair += kPairs) {
+            const bool mine = kPairs > 1 || (wave >> 1) == pair;
             __syncthreads();
-            if (wave == 2 * pair) {
+            if (mine && !(wave & 1)) {
 #pragma unroll
-                for (int r = 0; r < kPfRtw; ++r)
+                for (int r = 0; r < kRtw; ++r)
 #pragma unroll
                     for (int t = 0; t < NTT; ++t)
 #pragma unroll
                         for (int i = 0; i < 4; ++i) gbuf[(16 * r + 4 * q + i) * kPfGPitch + 16 * t + jt] = acc[r][t][i];
             }
             __syncthreads();
-            if (wave == 2 * pair + 1) {
+            if (mine && (wave & 1)) {
                 constexpr bool round_gu = FORM & kPfRoundGU, scale_h = FORM & kPfScaleH;
 #pragma unroll
                 for (int t = 0; t < NTT; ++t) {
@@ -845,7 +912,7 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int 
                         float wr = 1.0f;
                         if constexpr (scale_h) wr = a.w_row[row0 + tok];
 #pragma unroll
-                        for (int r = 0; r < kPfRtw; ++r) {
+                        for (int r = 0; r < kRtw; ++r) {
                             float hv[4];
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
@@ -872,7 +939,7 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int 
             const int tok = 16 * t + jt;
             if (tok < n) {
 #pragma unroll
-                for (int r = 0; r < kPfRtw; ++r)
+                for (int r = 0; r < kRtw; ++r)
                     *(float4 *)(a.out32 + (size_t)(row0 + tok) * a.R + rbase + 16 * r + 4 * q) =
                         make_float4(acc[r][t][0], acc[r][t][1], acc[r][t][2], acc[r][t][3]);
             }
@@ -883,7 +950,7 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int 
             const int tok = 16 * t + jt;
             if (tok < n) {
 #pragma unroll
-                for (int r = 0; r < kPfRtw; ++r) {
+                for (int r = 0; r < kRtw; ++r) {
                     uint2 v;
                     v.x = f32_to_bf16_rne(acc[r][t][0]) | (f32_to_bf16_rne(acc[r][t][1]) << 16);
                     v.y = f32_to_bf16_rne(acc[r][t][2]) | (f32_to_bf16_rne(acc[r][t][3]) << 16);
@@ -895,16 +962,16 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared &sh, int 
 }
 
 template <int MODE, class WP, int FORM>   // MODE 0: gate/up -> h, 1: down -> y; FORM: kPf* rounding forms
-__global__ void __launch_bounds__(64 * kPfWaves, 2) prefill_kernel(PfArgs a) {
-    __shared__ PfShared sh;
-    // workgroups are dispatched to the XCDs round-robin: all workgroups of one block go to the same XCD (block
-    // g on XCD g % 8), so the block's activation rows are fetched into one L2 and read there by every workgroup
+__global__ void __launch_bounds__(64 * WP::kWaves, WP::kCols == 128 ? kPfBPerSimd : 2) prefill_kernel(PfArgs a) {
+    __shared__ PfShared<WP> sh;
+    // Workgroups are dispatched to the XCDs round-robin.  The blocks, in launch order (most token tiles first), are
+    // dealt to the XCDs eight at a time, all workgroups of a block on one XCD, so the block's activation rows are
+    // fetched into one L2 and read there by every workgroup.  The tasks of the blocks left over are dealt one by one:
+    // whole, they would give some XCDs a block more than the others, an eighth of a launch of 64 blocks.
     // A launch runs n_blocks x RBG tasks on P resident workgroups.  The tasks of the last, partial round (its
     // blocks' tasks: the last sb blocks) are split along K into np pieces each, so that they spread over the slots
-    // that free up: np = P / (their tasks), at most kPfMaxPieces and at most the row's super tiles.  Their
-    // workgroups follow the unsplit tasks' (which keep the XCD mapping above and skip the split blocks).
+    // that free up: np = P / (their tasks), at most kPfMaxPieces and at most the row's super tiles.
     const int nb = *a.n_blocks;
-    const int wpad = (nb + kXcds - 1) / kXcds * kXcds * a.RBG;
     int sb = 0, np = 1;
     if constexpr (WP::kSplit) {
         const int r = (nb * a.RBG) % a.P;
@@ -915,21 +982,29 @@ __global__ void __launch_bounds__(64 * kPfWaves, 2) prefill_kernel(PfArgs a) {
             if (np < 2) np = 1, sb = 0;
         }
     }
-    int g, rbg, piece = 0, sti = 0, pieces = 1;
-    if ((int)blockIdx.x < wpad) {
-        const int xcd = blockIdx.x % kXcds, li = blockIdx.x / kXcds;
-        g = (li / a.RBG) * kXcds + xcd;
+    const int xcd = blockIdx.x % kXcds, li = blockIdx.x / kXcds;
+    const int rounds = (nb - sb) / kXcds;               // blocks per XCD dealt whole
+    int o, rbg, piece = 0, sti = 0, pieces = 1;
+    if (li < rounds * a.RBG) {
+        o = (li / a.RBG) * kXcds + xcd;
         rbg = li % a.RBG;
-        if (g >= nb - sb) return;                       // past the last block, or a split block
     } else {
-        const int i = blockIdx.x - wpad;
-        if (i >= np * sb * a.RBG) return;
-        sti = i / np;
-        piece = i - sti * np;
-        pieces = np;
-        g = nb - sb + sti / a.RBG;
-        rbg = sti % a.RBG;
+        const int t = (li - rounds * a.RBG) * kXcds + xcd;
+        const int whole = (nb - sb - rounds * kXcds) * a.RBG;
+        if (t < whole) {
+            o = rounds * kXcds + t / a.RBG;
+            rbg = t % a.RBG;
+        } else {
+            const int i = t - whole;
+            if (i >= np * sb * a.RBG) return;           // past the last task
+            sti = i / np;
+            piece = i - sti * np;
+            pieces = np;
+            o = nb - sb + sti / a.RBG;
+            rbg = sti % a.RBG;
+        }
     }
+    const int g = __builtin_amdgcn_readfirstlane(a.blk_order[o]);
     const int e = __builtin_amdgcn_readfirstlane(a.blk_expert[g]);
     const int n = __builtin_amdgcn_readfirstlane(a.blk_n[g]);
     // the format's LDS table (published by the barrier after the row offsets)
@@ -938,20 +1013,20 @@ __global__ void __launch_bounds__(64 * kPfWaves, 2) prefill_kernel(PfArgs a) {
                (uint32_t)__builtin_bit_cast(unsigned short, (_Float16)hi) << 16;
     };
     if constexpr (std::is_same<WP, PfIq3>::value) {
-        for (int i = threadIdx.x; i < 512; i += 64 * kPfWaves) {
+        for (int i = threadIdx.x; i < 512; i += 64 * WP::kWaves) {
             const uint32_t v = kPfGrid[i];
-            sh.iq3grid[i] = make_uint2(f16_pair((float)(v & 255u), (float)((v >> 8) & 255u)),
+            sh.tab.iq3grid[i] = make_uint2(f16_pair((float)(v & 255u), (float)((v >> 8) & 255u)),
                                        f16_pair((float)((v >> 16) & 255u), (float)(v >> 24)));
         }
     }
     if constexpr (std::is_same<WP, PfIq2>::value) {
         // levels 8, 25, 43 -> codes 0, 1, 2
-        for (int i = threadIdx.x; i < 1024; i += 64 * kPfWaves)
-            sh.iq2code[i] = make_uint2((kPfGrid2[2 * i] >> 4) & 0x03030303u, (kPfGrid2[2 * i + 1] >> 4) & 0x03030303u);
+        for (int i = threadIdx.x; i < 1024; i += 64 * WP::kWaves)
+            sh.tab.iq2code[i] = make_uint2((kPfGrid2[2 * i] >> 4) & 0x03030303u, (kPfGrid2[2 * i + 1] >> 4) & 0x03030303u);
     }
     if constexpr (std::is_same<WP, PfIq4>::value) {
-        for (int i = threadIdx.x; i < 256; i += 64 * kPfWaves)
-            sh.iq4pair[i] = f16_pair((float)kPfKv[i & 15], (float)kPfKv[i >> 4]);
+        for (int i = threadIdx.x; i < 256; i += 64 * WP::kWaves)
+            sh.tab.iq4pair[i] = f16_pair((float)kPfKv[i & 15], (float)kPfKv[i >> 4]);
     }
     switch ((n + 15) >> 4) {
         case 1: prefill_body<MODE, 1, WP, FORM>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
@@ -965,7 +1040,7 @@ __global__ void __launch_bounds__(64 * kPfWaves, 2) prefill_kernel(PfArgs a) {
 // Launches prefill_kernel<MODE, *, FORM> for the table format qtype (MI_QT_*) on grid workgroups.
 template <int MODE, int FORM>
 int launch_prefill(int qtype, dim3 grid, hipStream_t s, const PfArgs &a) {
-    const dim3 block(64 * kPfWaves);
+    const dim3 block(64 * (qtype == MI_QT_CB3 ? kPfWaves : kPfBWaves));
     switch (qtype) {
         case MI_QT_IQ3_S: hipLaunchKernelGGL((prefill_kernel<MODE, PfIq3, FORM>), grid, block, 0, s, a); break;
         case MI_QT_IQ4_XS: hipLaunchKernelGGL((prefill_kernel<MODE, PfIq4, FORM>), grid, block, 0, s, a); break;
