@@ -410,7 +410,7 @@ size_t mi_mlp_many_workspace(int32_t B, int32_t D, int32_t I);
  * split counts and row tiles of the decode launch families (S1, S2, FS1, FS2, SMV, each with _RTW and _AL; MS1, MS2,
  * CS1, CS2 with _RTW; MGMAX), launch-family switches (CUSTREAM, CUMULTI, PERSIST_ABOVE, FUSE_SWIGLU, CU_FORM_H), the
  * one-launch decode's poll limit (SPIN_LIMIT), the int8 split plan (I8S, I8_WAVES, I8_FUSE) and the many-token MLP's
- * splits and token tile (DG_S1, DG_S2, DG_NT).  Overrides change
+ * splits and token tile (DG_S1, DG_S2, DG_NT) and the prefill's wide blocks (PF_WIDE).  Overrides change
  * launch shapes and summation orders, never the result beyond f32 rounding; workspace sizes follow them, so set them
  * before sizing a workspace.  Not synchronised with calls running on other host threads.
  */

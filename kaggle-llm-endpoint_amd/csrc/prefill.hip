@@ -13,6 +13,7 @@
 #include <climits>
 
 #include "prefill_gemm.h"
+#include "tuning.h"
 
 namespace mi {
 constexpr int kPlanThreads = 1024;
@@ -30,6 +31,7 @@ struct PlanOut {
     int32_t *row_slot;     // [T * kk] sorted row of every (token, slot); -1 for an expert id outside [0, E)
     int32_t *blk_n;        // [G]   rows of every block that are not padding (NULL: not written)
     int32_t *blk_order;    // [G]   blocks in launch order: most token tiles first (NULL: not written)
+    int even;              // an expert's blocks share its rows evenly, in multiples of 16 (0: whole blocks of tm first)
     int merge_dups;        // w_row of the first slot of a token's expert = the sum of that token's weights of the
                            // expert in column order, 0 for its later slots (the sweeps' summed routing weight)
     uint32_t *cnt;         // [n_cnt] the grouped GEMMs' split-task counters, zeroed here (NULL: none)
@@ -103,7 +105,8 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
     __shared__ int cnt[kPlanMaxE], bend[kPlanMaxE], rbase[kPlanMaxE];
     __shared__ unsigned long long lanes[kPlanWaves][kPlanMaskE];   // pass 2: lanes of every id in this step
     __shared__ int wsum[kPlanWaves];
-    __shared__ int ntile[kPfTT + 1];              // blocks of every token tile count, then the first position of each
+    __shared__ int per[kPlanMaxE];                // rows per block of every expert (the last one fewer)
+    __shared__ int ntile[kPfWideTT + 1];           // blocks of every token tile count, then the first position of each
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kk = k + (shared >= 0 ? 1 : 0);
     const int S = T * kk;
@@ -187,11 +190,13 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
     if (tid < kPlanMaxE) {
         bend[tid] = incl;
         rbase[tid] = (incl - nb_own) * tm;
+        // evenly: at most tm (a multiple of 16 then), and the nb_own - 1 blocks before the last hold fewer than cnt rows
+        per[tid] = p.even && nb_own > 0 ? ((cnt[tid] + nb_own - 1) / nb_own + 15) / 16 * 16 : tm;
     }
     __syncthreads();
     const int n_blocks = bend[kPlanMaxE - 1];
     if (tid == 0) *p.n_blocks = n_blocks;
-    if (tid <= kPfTT) ntile[tid] = 0;
+    if (tid <= kPfWideTT) ntile[tid] = 0;
     for (int i = tid; i < p.n_cnt; i += kPlanThreads) p.cnt[i] = 0u;
     vm_wait<0>();                              // this wavefront's padding stores are done ...
     __syncthreads();                            // ... and every other wavefront's
@@ -217,7 +222,8 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
             const int below = __popcll(m & ((1ull << lane) - 1ull));
             int row = -1;
             if (valid) {
-                row = rbase[e] + cntw[e][wave] + below;
+                const int pos = cntw[e][wave] + below, b = pos / per[e];
+                row = rbase[e] + b * tm + pos - b * per[e];
                 p.tok_row[row] = treg[r];
                 p.w_row[row] = wreg[r];
             }
@@ -254,7 +260,7 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
             }
             e = lo;
             const int nb = (cnt[e] + tm - 1) / tm;
-            n = min(tm, cnt[e] - (g - (bend[e] - nb)) * tm);
+            n = min(per[e], cnt[e] - (g - (bend[e] - nb)) * per[e]);
         }
         p.blk_expert[g] = e;
         if (p.blk_n) p.blk_n[g] = n;
@@ -267,7 +273,7 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
     __syncthreads();
     if (tid == 0) {
         int at = 0;
-        for (int c = kPfTT; c > 0; --c) {
+        for (int c = kPfWideTT; c > 0; --c) {
             const int m = ntile[c];
             ntile[c] = at;
             at += m;
@@ -403,18 +409,18 @@ struct PfLayout {
     size_t off_be, off_nb, off_bn, off_bo, off_tr, off_wr, off_rs, off_h, off_y, off_part, off_cnt, total;
 };
 
-// Workgroups of a block-format GEMM launch resident at once: kPfBPerSimd per CU, one wavefront of each on every SIMD.
+// Workgroups of a block-format GEMM launch resident at once: pf_per_simd per CU, one wavefront of each on every SIMD.
 // The launches split their last round's tasks by it (prefill_gemm.h).
-static int pf_slots() {
-    static int slots = 0;
-    if (!slots) {
-        int dev = 0, cus = 0;
+static int pf_slots(int tt) {
+    static int cus = 0;
+    if (!cus) {
+        int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
-        slots = kPfBPerSimd * cus;
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        cus = n;
     }
-    return slots;
+    return pf_per_simd(tt) * cus;
 }
 
 static size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -422,11 +428,12 @@ static size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
 // y holds bf16 rows for the ragged and XLA-gather forms, f32 rows for the sweeps
 static bool pf_y32(int combine) { return combine == MI_COMBINE_SWEEP || combine == MI_COMBINE_XLA_SWEEP; }
 
-static PfLayout pf_layout(int T, int kk, int E, int I, int D, bool y32) {
+static PfLayout pf_layout(int T, int kk, int E, int I, int D, bool y32, int tt) {
+    const int tm = 16 * tt;
     PfLayout L{};
     L.S = T * kk;
-    L.G = (L.S + kPfTm - 1) / kPfTm + E;
-    L.Rp = (long long)L.G * kPfTm;
+    L.G = (L.S + tm - 1) / tm + E;
+    L.Rp = (long long)L.G * tm;
     size_t o = 0;
     L.off_be = o; o = al256(o + 4 * (size_t)L.G);
     L.off_nb = o; o = al256(o + 4);
@@ -437,8 +444,8 @@ static PfLayout pf_layout(int T, int kk, int E, int I, int D, bool y32) {
     L.off_rs = o; o = al256(o + 4 * (size_t)L.S);
     L.off_h = o; o = al256(o + 2 * (size_t)L.Rp * I);
     L.off_y = o; o = al256(o + (y32 ? 4 : 2) * (size_t)L.Rp * D);
-    L.P = pf_slots();
-    L.off_part = o; o = al256(o + (size_t)L.P * kPfPartBytes);
+    L.P = pf_slots(tt);
+    L.off_part = o; o = al256(o + (size_t)L.P * pf_part_bytes(tt));
     L.off_cnt = o; o = al256(o + 4 * (size_t)L.P);
     L.total = o;
     return L;
@@ -542,10 +549,25 @@ static bool plan_sizes_ok(long long T, long long kk, long long E, long long tm) 
 }
 
 // The activation buffers are addressed with 32-bit byte offsets: x [T, D], h [Rp, I] and y [Rp, D] stay below 2 GiB.
-static bool pf_bytes_ok(long long T, long long kk, long long E, long long I, long long D) {
-    const long long Rp = ((T * kk + kPfTm - 1) / kPfTm + E) * kPfTm;
+static bool pf_bytes_ok(long long T, long long kk, long long E, long long I, long long D, int tt) {
+    const long long tm = 16 * tt, Rp = ((T * kk + tm - 1) / tm + E) * tm;
     const long long lim = 1ll << 31;
     return T * D * 2 < lim && Rp * I * 2 < lim && Rp * D * 2 < lim;
+}
+
+// Token tiles per block of a call's plan: wide blocks (block formats only) where they cut an expert of the mean row
+// count into fewer blocks, i.e. decode its weights fewer times: above 80 rows, except 129..160 (two blocks either way).
+// With the same number the narrow launches' third wavefront per SIMD wins.  D 6144, I 2048, 64 experts, top-8, narrow /
+// wide: IQ3_S 512 tokens (64 rows) 599 / 635 us, 700 (88) 889 / 721, 900 (113) 1033 / 852, 1200 (150) 1247 / 1303, 1999
+// (250) 1996 / 1734; Q2_K + Q3_K the same way.
+static int pf_tt(const mi_table *gate, const mi_table *down, int T, int kk) {
+    const int E = gate->n_experts;
+    if (gate->qtype == MI_QT_CB3 || down->qtype == MI_QT_CB3) return kPfTT;
+    const long long S = (long long)T * kk;
+    const auto blocks = [&](long long tm) { return (S + tm * E - 1) / (tm * E); };      // of an expert of S / E rows
+    if (!tuning(kTunePfWide, blocks(16 * kPfWideTT) < blocks(16 * kPfTT))) return kPfTT;
+    return plan_sizes_ok(T, kk, E, 16 * kPfWideTT) && pf_bytes_ok(T, kk, E, gate->rows, down->rows, kPfWideTT) ? kPfWideTT
+                                                                                                             : kPfTT;
 }
 
 static int launch_plan(const int32_t *idx, const float *w, int T, int k, int shared, int E, int tm, PlanOut p,
@@ -567,7 +589,7 @@ int mi_ragged_plan(const int32_t *idx, const float *w, int32_t T, int32_t k, int
     if (T <= 0 || k <= 0) return MI_ERR_TOKENS;
     if (E <= 0 || E > kPlanMaxE || tm <= 0 || tm > 65536) return MI_ERR_ARG;
     if (!plan_sizes_ok(T, k, E, tm)) return MI_ERR_TOKENS;
-    PlanOut p{blk_expert, n_blocks, tok_row, w_row, row_slot, nullptr, nullptr, 0, nullptr, 0};
+    PlanOut p{blk_expert, n_blocks, tok_row, w_row, row_slot, nullptr, nullptr, 0, 0, nullptr, 0};
     return launch_plan(idx, w, T, k, -1, E, tm, p, (hipStream_t)stream);
 }
 
@@ -575,9 +597,9 @@ size_t mi_moe_prefill_form_workspace(const mi_table *gate, const mi_table *down,
                                      int32_t shared_expert, int32_t combine) {
     if (!gate || !down || k <= 0 || combine < MI_COMBINE_MATMUL || combine > MI_COMBINE_XLA_SWEEP) return 0;
     const int kk = k + (shared_expert >= 0 ? 1 : 0);
-    if (!plan_sizes_ok(T, kk, gate->n_experts, kPfTm) || !pf_bytes_ok(T, kk, gate->n_experts, gate->rows, down->rows))
-        return 0;
-    return pf_layout(T, kk, gate->n_experts, gate->rows, down->rows, pf_y32(combine)).total;
+    const int E = gate->n_experts, tt = pf_tt(gate, down, T, kk);
+    if (!plan_sizes_ok(T, kk, E, 16 * tt) || !pf_bytes_ok(T, kk, E, gate->rows, down->rows, tt)) return 0;
+    return pf_layout(T, kk, E, gate->rows, down->rows, pf_y32(combine), tt).total;
 }
 
 size_t mi_moe_prefill_workspace(const mi_table *gate, const mi_table *down, int32_t T, int32_t k,
@@ -606,11 +628,12 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     if (T <= 0 || k <= 0) return MI_ERR_TOKENS;
     if (shared_expert >= E || shared_expert < -1) return MI_ERR_ARG;
     const int kk = k + (shared_expert >= 0 ? 1 : 0);
-    if (!plan_sizes_ok(T, kk, E, kPfTm) || !pf_bytes_ok(T, kk, E, I, D)) return MI_ERR_TOKENS;
+    const int tt = pf_tt(gate, down, T, kk);
+    if (!plan_sizes_ok(T, kk, E, 16 * tt) || !pf_bytes_ok(T, kk, E, I, D, tt)) return MI_ERR_TOKENS;
     if (!(limit > 0.0f) || combine < MI_COMBINE_MATMUL || combine > MI_COMBINE_XLA_SWEEP) return MI_ERR_ARG;
     if (combine == MI_COMBINE_XLA_SWEEP && chunk <= 0) return MI_ERR_ARG;
     const bool y32 = pf_y32(combine);
-    const PfLayout L = pf_layout(T, kk, E, I, D, y32);
+    const PfLayout L = pf_layout(T, kk, E, I, D, y32, tt);
     if (!workspace || workspace_bytes < L.total) return MI_ERR_WORKSPACE;
     char *ws = (char *)workspace;
     hipStream_t s = (hipStream_t)stream;
@@ -622,11 +645,12 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     p.tok_row = (int32_t *)(ws + L.off_tr);
     p.w_row = (float *)(ws + L.off_wr);
     p.row_slot = (int32_t *)(ws + L.off_rs);
+    p.even = 1;
     p.merge_dups = y32;
     p.cnt = (uint32_t *)(ws + L.off_cnt);
     p.n_cnt = L.P;
     uint16_t *h = (uint16_t *)(ws + L.off_h), *y = (uint16_t *)(ws + L.off_y);
-    if ((st = launch_plan(idx, w, T, k, shared_expert, E, kPfTm, p, s))) return st;
+    if ((st = launch_plan(idx, w, T, k, shared_expert, E, 16 * tt, p, s))) return st;
 
     PfArgs a{};
     if (gate->qtype == MI_QT_IQ3_S) {
@@ -659,6 +683,7 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     a.limit = limit;
     a.RBG = gate->qtype == MI_QT_CB3 ? I / 128 : I / (8 * kPfBWaves * kPfBRtw);
     a.w_row = p.w_row;
+    a.wide = tt == kPfWideTT;
     a.P = L.P;
     a.part = (float *)(ws + L.off_part);
     a.cnt = p.cnt;

@@ -31,17 +31,21 @@ static __constant__ int8_t kPfKv[16] = {
 };
 
 constexpr int kPfTT = 5;                   // token tiles of 16 rows per block
-constexpr int kPfTm = 16 * kPfTT;          // rows per block of the prefill's own plan
+constexpr int kPfWideTT = 8;               // ... of the wide launches (block formats, many rows per expert)
 constexpr int kPfWaves = 4;                // CB3: wavefronts per workgroup ...
 constexpr int kPfRtw = 4;                  // ... and row tiles per wavefront (64 weight rows)
 // The block formats: 128 rows per workgroup, 4 wavefronts of 32 rows in at most 168 registers and 49 KB of LDS, so that
 // three wavefronts per SIMD cover each other's table gathers, barriers and loads.  IQ2_S + IQ4_XS layer, D 6144, I 2048,
 // against two wavefronts of 64 rows (256 registers, 77 KB) with the same decoders: 27 tokens 319 -> 292 us, 512 tokens
 // the same; in launch order by token tiles with the last blocks' tasks dealt singly 285 and 531 (from 541)
-constexpr int kPfBWaves = 4, kPfBRtw = 2, kPfBPerSimd = 3;
+//
+// The wide launches decode a weight once for up to 128 rows instead of 80, with two wavefronts per SIMD (acc and staging
+// of 8 token tiles): fewer decodes where an expert's rows fill such blocks, fewer wavefronts where they do not.
+constexpr int kPfBWaves = 4, kPfBRtw = 2;
+constexpr int pf_per_simd(int tt) { return tt > kPfTT ? 2 : 3; }
 constexpr int kPfXPitch = 88;              // dwords per staged activation row of one column tile (80 + 8: the
                                            // fastest pitch for this read pattern on gfx950, measured)
-constexpr int kPfGPitch = kPfTm + 4;       // floats per row of the gate/up epilogue's exchange (skewed banks)
+constexpr int pf_gpitch(int tt) { return 16 * tt + 4; }   // floats per row of the gate/up epilogue's exchange (skewed banks)
 constexpr int kXcds = 8;                   // accelerator complex dies of MI355X (one L2 each)
 constexpr uint32_t kXOut = 0x80000000u;    // activation offset past every buffer's byte range (reads zero)
 
@@ -62,15 +66,16 @@ struct PfArgs {
     int RBG;                               // workgroups per block
     const float *w_row;                    // gate/up with kPfScaleH: the plan's routing weight of every row
     float *out32;                          // down with kPfY32: y [Rp, R] in f32
+    int wide;                              // blocks of kPfWideTT token tiles
     int P;                                 // workgroups resident at once over the chip
-    float *part;                           // split tasks' piece sums: P x kPfPartBytes
+    float *part;                           // split tasks' piece sums: P x pf_part_bytes(TT)
     uint32_t *cnt;                         // split tasks' piece counters: P, zero between launches
 };
 
 // A task of the launch's last, partial round is split along K into pieces (at most kPfMaxPieces, whole super tiles
-// each); a piece stores its accumulators here (kPfPartBytes per workgroup).
+// each); a piece stores its accumulators here (pf_part_bytes per workgroup).
 constexpr int kPfMaxPieces = 4;
-constexpr int kPfPartBytes = kPfBWaves * kPfBRtw * kPfTT * 64 * 16;
+constexpr int pf_part_bytes(int tt) { return kPfBWaves * kPfBRtw * tt * 64 * 16; }
 
 // Rounding forms of the epilogues (FORM, a compile-time set; the ragged kernels use none):
 constexpr int kPfRoundGU = 1;   // gate/up: g and u rounded to bf16 before the SwiGLU (the XLA einsums' bf16 outputs)
@@ -156,13 +161,13 @@ __device__ __forceinline__ void pf_ctile(const Cb3Wave &w, PfRegs &s, int st, co
 // chunk of step j is act_chunk(q) plus a constant of j on other bits, so an exclusive or with that constant finds it.
 constexpr int kPfXRow = 256;
 
-template <class WP>
+template <class WP, int TT>
 struct PfShared {
-    typename WP::Table tab;                      // the format's table, or CB3's codebook slots
+    alignas(16) typename WP::Table tab;                      // the format's table, or CB3's codebook slots
     // column tiles ct (even/odd) of the block's rows, double-buffered; gate/up epilogue: gate accumulators
-    static constexpr int kXBuf = kPfTm * (WP::kCols == 128 ? kPfXRow / 4 : kPfXPitch);
-    uint32_t xs[2][kXBuf];
-    uint32_t xrowoff[kPfTm];                     // byte offset of every row's activations, or kXOut
+    static constexpr int kXBuf = 16 * TT * (WP::kCols == 128 ? kPfXRow / 4 : kPfXPitch);
+    alignas(16) uint32_t xs[2][kXBuf];           // read and written 16 bytes at a time
+    uint32_t xrowoff[16 * TT];                     // byte offset of every row's activations, or kXOut
     int last;                                    // split task: this workgroup's piece arrived last
 };
 
@@ -731,13 +736,14 @@ struct PfIq4 {
 // One workgroup: block g (expert e, rows row0 .. row0 + n - 1, NTT = ceil(n / 16) token tiles), row range rbg.
 // piece / np: the workgroup runs super tiles [piece n_st / np, (piece + 1) n_st / np) of the task (np == 1: all of
 // them); sti: the split task's index among the launch's split tasks (counter and piece sums).
-template <int MODE, int NTT, class WP, int FORM>
-__device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP> &sh, int g, int rbg, int e, int n, int piece,
+template <int MODE, int NTT, class WP, int FORM, int TT>
+__device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP, TT> &sh, int g, int rbg, int e, int n, int piece,
                                              int np, int sti) {
     uint32_t *xs = &sh.xs[0][0], *xrowoff = sh.xrowoff;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int row0 = g * kPfTm;
+    constexpr int kTm = 16 * TT;                         // rows per block of the plan
+    const int row0 = g * kTm;
     const int mat = MODE == 0 ? (wave & 1) : 0;
     constexpr int kRtw = WP::kRtw, kWaves = WP::kWaves;
     constexpr bool kBlock = WP::kCols == 128;             // a block format
@@ -758,11 +764,11 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP> &sh, 
     // which reads zero
     constexpr int kXU = WP::kCols / 8;                        // 20 (CB3) or 16 (IQ3_S)
     constexpr int kXRows = (64 * kWaves) / kXU;               // 12 or 32
-    constexpr int kXBuf = PfShared<WP>::kXBuf;                // dwords per tile buffer
+    constexpr int kXBuf = PfShared<WP, TT>::kXBuf;                // dwords per tile buffer
     constexpr int kXJ = (16 * NTT + kXRows - 1) / kXRows;
     const __amdgpu_buffer_rsrc_t xbuf =
         __builtin_amdgcn_make_buffer_rsrc((void *)a.x, (short)0, (int)a.x_bytes, kBufferWord3);
-    if (tid < kPfTm) {
+    if (tid < kTm) {
         uint32_t o = kXOut;
         if (tid < n) o = (uint32_t)(a.gather ? a.tok_row[row0 + tid] : row0 + tid) * (uint32_t)a.K * 2u;
         xrowoff[tid] = o;
@@ -857,8 +863,8 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP> &sh, 
             __builtin_amdgcn_make_buffer_rsrc((void *)a.part, (short)0, 0x7fffffff, kBufferWord3);
         const uint32_t lane_off = 16u * (uint32_t)lane;
         auto part_off = [&](int pc, int r, int t) {
-            return (uint32_t)(sti * np + pc) * (uint32_t)kPfPartBytes +
-                   (uint32_t)((wave * kRtw + r) * kPfTT + t) * 1024u + lane_off;
+            return (uint32_t)(sti * np + pc) * (uint32_t)pf_part_bytes(TT) +
+                   (uint32_t)((wave * kRtw + r) * TT + t) * 1024u + lane_off;
         };
 #pragma unroll
         for (int r = 0; r < kRtw; ++r)
@@ -887,10 +893,10 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP> &sh, 
     // epilogue: lane (jt, q) holds rows 16 r + 4 q + i (i = 0..3) of the wavefront's 64 rows for tokens 16 t + jt
     const int rbase = rg * 16 * kRtw;
     if constexpr (MODE == 0) {
-        // gate accumulators of as many (gate, up) pairs as the activation buffers hold at once: [rows][kPfGPitch]
-        constexpr int kPairs = kBlock ? kWaves / 2 : 1;
-        static_assert(kPairs * 16 * kRtw * kPfGPitch <= 2 * kXBuf, "the exchange fits the tile buffers");
-        float *gbuf = (float *)xs + (kPairs > 1 ? (wave >> 1) * 16 * kRtw * kPfGPitch : 0);
+        // gate accumulators of as many (gate, up) pairs as the activation buffers hold at once: [rows][kGPitch]
+        constexpr int kPairs = kBlock ? kWaves / 2 : 1, kGPitch = pf_gpitch(TT);
+        static_assert(kPairs * 16 * kRtw * kGPitch <= 2 * kXBuf, "the exchange fits the tile buffers");
+        float *gbuf = (float *)xs + (kPairs > 1 ? (wave >> 1) * 16 * kRtw * kGPitch : 0);
         for (int pair = 0; pair < kWaves / 2; pair += kPairs) {
             const bool mine = kPairs > 1 || (wave >> 1) == pair;
             __syncthreads();
@@ -900,7 +906,7 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP> &sh, 
 #pragma unroll
                     for (int t = 0; t < NTT; ++t)
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) gbuf[(16 * r + 4 * q + i) * kPfGPitch + 16 * t + jt] = acc[r][t][i];
+                        for (int i = 0; i < 4; ++i) gbuf[(16 * r + 4 * q + i) * kGPitch + 16 * t + jt] = acc[r][t][i];
             }
             __syncthreads();
             if (mine && (wave & 1)) {
@@ -916,7 +922,7 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP> &sh, 
                             float hv[4];
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
-                                float gv = gbuf[(16 * r + 4 * q + i) * kPfGPitch + tok], uv = acc[r][t][i];
+                                float gv = gbuf[(16 * r + 4 * q + i) * kGPitch + tok], uv = acc[r][t][i];
                                 if constexpr (round_gu) {
                                     gv = round_bf16(gv);
                                     uv = round_bf16(uv);
@@ -961,9 +967,9 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP> &sh, 
     }
 }
 
-template <int MODE, class WP, int FORM>   // MODE 0: gate/up -> h, 1: down -> y; FORM: kPf* rounding forms
-__global__ void __launch_bounds__(64 * WP::kWaves, WP::kCols == 128 ? kPfBPerSimd : 2) prefill_kernel(PfArgs a) {
-    __shared__ PfShared<WP> sh;
+template <int MODE, class WP, int FORM, int TT>   // MODE 0: gate/up -> h, 1: down -> y; FORM: kPf* rounding forms
+__global__ void __launch_bounds__(64 * WP::kWaves, WP::kCols == 128 ? pf_per_simd(TT) : 2) prefill_kernel(PfArgs a) {
+    __shared__ PfShared<WP, TT> sh;
     // Workgroups are dispatched to the XCDs round-robin.  The blocks, in launch order (most token tiles first), are
     // dealt to the XCDs eight at a time, all workgroups of a block on one XCD, so the block's activation rows are
     // fetched into one L2 and read there by every workgroup.  The tasks of the blocks left over are dealt one by one:
@@ -1028,26 +1034,44 @@ __global__ void __launch_bounds__(64 * WP::kWaves, WP::kCols == 128 ? kPfBPerSim
         for (int i = threadIdx.x; i < 256; i += 64 * WP::kWaves)
             sh.tab.iq4pair[i] = f16_pair((float)kPfKv[i & 15], (float)kPfKv[i >> 4]);
     }
-    switch ((n + 15) >> 4) {
-        case 1: prefill_body<MODE, 1, WP, FORM>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
-        case 2: prefill_body<MODE, 2, WP, FORM>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
-        case 3: prefill_body<MODE, 3, WP, FORM>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
-        case 4: prefill_body<MODE, 4, WP, FORM>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
-        default: prefill_body<MODE, kPfTT, WP, FORM>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+    if constexpr (TT == kPfTT) {
+        switch ((n + 15) >> 4) {
+            case 1: prefill_body<MODE, 1, WP, FORM, TT>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+            case 2: prefill_body<MODE, 2, WP, FORM, TT>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+            case 3: prefill_body<MODE, 3, WP, FORM, TT>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+            case 4: prefill_body<MODE, 4, WP, FORM, TT>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+            default: prefill_body<MODE, 5, WP, FORM, TT>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+        }
+    } else {
+        switch ((n + 31) >> 5) {                        // even counts: rows past n are zeros
+            case 1: prefill_body<MODE, 2, WP, FORM, TT>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+            case 2: prefill_body<MODE, 4, WP, FORM, TT>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+            case 3: prefill_body<MODE, 6, WP, FORM, TT>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+            default: prefill_body<MODE, 8, WP, FORM, TT>(a, sh, g, rbg, e, n, piece, pieces, sti); break;
+        }
     }
 }
 
 // Launches prefill_kernel<MODE, *, FORM> for the table format qtype (MI_QT_*) on grid workgroups.
+template <int MODE, int FORM, class WP>
+void launch_prefill_block(dim3 grid, hipStream_t s, const PfArgs &a) {
+    if (a.wide)
+        hipLaunchKernelGGL((prefill_kernel<MODE, WP, FORM, kPfWideTT>), grid, dim3(64 * kPfBWaves), 0, s, a);
+    else
+        hipLaunchKernelGGL((prefill_kernel<MODE, WP, FORM, kPfTT>), grid, dim3(64 * kPfBWaves), 0, s, a);
+}
+
 template <int MODE, int FORM>
 int launch_prefill(int qtype, dim3 grid, hipStream_t s, const PfArgs &a) {
-    const dim3 block(64 * (qtype == MI_QT_CB3 ? kPfWaves : kPfBWaves));
     switch (qtype) {
-        case MI_QT_IQ3_S: hipLaunchKernelGGL((prefill_kernel<MODE, PfIq3, FORM>), grid, block, 0, s, a); break;
-        case MI_QT_IQ4_XS: hipLaunchKernelGGL((prefill_kernel<MODE, PfIq4, FORM>), grid, block, 0, s, a); break;
-        case MI_QT_IQ2_S: hipLaunchKernelGGL((prefill_kernel<MODE, PfIq2, FORM>), grid, block, 0, s, a); break;
-        case MI_QT_Q2_K: hipLaunchKernelGGL((prefill_kernel<MODE, PfKq<false>, FORM>), grid, block, 0, s, a); break;
-        case MI_QT_Q3_K: hipLaunchKernelGGL((prefill_kernel<MODE, PfKq<true>, FORM>), grid, block, 0, s, a); break;
-        case MI_QT_CB3: hipLaunchKernelGGL((prefill_kernel<MODE, PfCb3, FORM>), grid, block, 0, s, a); break;
+        case MI_QT_IQ3_S: launch_prefill_block<MODE, FORM, PfIq3>(grid, s, a); break;
+        case MI_QT_IQ4_XS: launch_prefill_block<MODE, FORM, PfIq4>(grid, s, a); break;
+        case MI_QT_IQ2_S: launch_prefill_block<MODE, FORM, PfIq2>(grid, s, a); break;
+        case MI_QT_Q2_K: launch_prefill_block<MODE, FORM, PfKq<false>>(grid, s, a); break;
+        case MI_QT_Q3_K: launch_prefill_block<MODE, FORM, PfKq<true>>(grid, s, a); break;
+        case MI_QT_CB3:
+            hipLaunchKernelGGL((prefill_kernel<MODE, PfCb3, FORM, kPfTT>), grid, dim3(64 * kPfWaves), 0, s, a);
+            break;
         default: return MI_ERR_QTYPE;
     }
     return hipGetLastError() == hipSuccess ? MI_OK : MI_ERR_LAUNCH;

@@ -17,6 +17,7 @@ enum Knob : int {
     kTuneCustream, kTuneCumulti, kTunePersistAbove, kTuneFuseSwiglu, kTuneCuFormH, kTuneSpinLimit, kTuneCuCombine,
     kTuneI8S, kTuneI8Waves, kTuneI8Fuse,
     kTuneDgS1, kTuneDgS2, kTuneDgNt,         // many-token MLP: gate/up and down splits, token tiles per wavefront
+    kTunePfWide,                             // prefill: 1 wide blocks, 0 narrow ones
     kTuneCount
 };
 

@@ -31,6 +31,7 @@ const Entry kNames[] = {
     {"CU_COMBINE", kTuneCuCombine},
     {"I8S", kTuneI8S}, {"I8_WAVES", kTuneI8Waves}, {"I8_FUSE", kTuneI8Fuse},
     {"DG_S1", kTuneDgS1}, {"DG_S2", kTuneDgS2}, {"DG_NT", kTuneDgNt},
+    {"PF_WIDE", kTunePfWide},
 };
 static_assert(sizeof(kNames) / sizeof(kNames[0]) == kTuneCount, "every knob has a name");
 
