@@ -10,6 +10,7 @@
 // The rounding points are the reference's: bf16 activations, bf16 weights (CB3 centroids are bf16 already; IQ2_S /
 // IQ3_S / IQ4_XS level * scale rounded once), f32 accumulation, h and y rounded to bf16, routing weights rounded to
 // bf16 by the matmul combine; the other branches' forms as mi_moe_prefill_form states them.
+#include <algorithm>
 #include <climits>
 
 #include "prefill_gemm.h"
@@ -409,9 +410,9 @@ struct PfLayout {
     size_t off_be, off_nb, off_bn, off_bo, off_tr, off_wr, off_rs, off_h, off_y, off_part, off_cnt, total;
 };
 
-// Workgroups of a block-format GEMM launch resident at once: pf_per_simd per CU, one wavefront of each on every SIMD.
-// The launches split their last round's tasks by it (prefill_gemm.h).
-static int pf_slots(int tt) {
+// Workgroups of a GEMM launch resident at once: pf_per_simd per CU, one wavefront of each on every SIMD.  The launches
+// split their last round's tasks by it (prefill_gemm.h).
+static int pf_slots(int tt, bool block) {
     static int cus = 0;
     if (!cus) {
         int dev = 0, n = 0;
@@ -420,7 +421,7 @@ static int pf_slots(int tt) {
             n = 256;
         cus = n;
     }
-    return pf_per_simd(tt) * cus;
+    return pf_per_simd(tt, block) * cus;
 }
 
 static size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -444,8 +445,10 @@ static PfLayout pf_layout(int T, int kk, int E, int I, int D, bool y32, int tt) 
     L.off_rs = o; o = al256(o + 4 * (size_t)L.S);
     L.off_h = o; o = al256(o + 2 * (size_t)L.Rp * I);
     L.off_y = o; o = al256(o + (y32 ? 4 : 2) * (size_t)L.Rp * D);
-    L.P = pf_slots(tt);
-    L.off_part = o; o = al256(o + (size_t)L.P * pf_part_bytes(tt));
+    // either GEMM may be of a block format or CB3
+    L.P = std::max(pf_slots(tt, true), pf_slots(tt, false));
+    L.off_part = o; o = al256(o + std::max((size_t)pf_slots(tt, true) * pf_part_bytes(tt, true),
+                                           (size_t)pf_slots(tt, false) * pf_part_bytes(tt, false)));
     L.off_cnt = o; o = al256(o + 4 * (size_t)L.P);
     L.total = o;
     return L;
@@ -684,7 +687,7 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     a.RBG = gate->qtype == MI_QT_CB3 ? I / 128 : I / (8 * kPfBWaves * kPfBRtw);
     a.w_row = p.w_row;
     a.wide = tt == kPfWideTT;
-    a.P = L.P;
+    a.P = pf_slots(tt, gate->qtype != MI_QT_CB3);
     a.part = (float *)(ws + L.off_part);
     a.cnt = p.cnt;
     // every block's tasks and at most P pieces of split ones, in whole XCD rounds
@@ -708,6 +711,7 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     b.gather = 0;
     b.out = y;
     b.RBG = down->qtype == MI_QT_CB3 ? D / 256 : D / (16 * kPfBWaves * kPfBRtw);
+    b.P = pf_slots(tt, down->qtype != MI_QT_CB3);
     b.out32 = (float *)y;
     const dim3 gdn(g8 * b.RBG + L.P);
     if ((st = y32 ? launch_prefill_1_4(down->qtype, gdn, s, b) : launch_prefill_1_0(down->qtype, gdn, s, b))) return st;

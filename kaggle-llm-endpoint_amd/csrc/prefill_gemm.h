@@ -42,7 +42,7 @@ constexpr int kPfRtw = 4;                  // ... and row tiles per wavefront (6
 // The wide launches decode a weight once for up to 128 rows instead of 80, with two wavefronts per SIMD (acc and staging
 // of 8 token tiles): fewer decodes where an expert's rows fill such blocks, fewer wavefronts where they do not.
 constexpr int kPfBWaves = 4, kPfBRtw = 2;
-constexpr int pf_per_simd(int tt) { return tt > kPfTT ? 2 : 3; }
+constexpr int pf_per_simd(int tt, bool block) { return !block || tt > kPfTT ? 2 : 3; }
 constexpr int kPfXPitch = 88;              // dwords per staged activation row of one column tile (80 + 8: the
                                            // fastest pitch for this read pattern on gfx950, measured)
 constexpr int pf_gpitch(int tt) { return 16 * tt + 4; }   // floats per row of the gate/up epilogue's exchange (skewed banks)
@@ -68,14 +68,14 @@ struct PfArgs {
     float *out32;                          // down with kPfY32: y [Rp, R] in f32
     int wide;                              // blocks of kPfWideTT token tiles
     int P;                                 // workgroups resident at once over the chip
-    float *part;                           // split tasks' piece sums: P x pf_part_bytes(TT)
+    float *part;                           // split tasks' piece sums: P x pf_part_bytes
     uint32_t *cnt;                         // split tasks' piece counters: P, zero between launches
 };
 
 // A task of the launch's last, partial round is split along K into pieces (at most kPfMaxPieces, whole super tiles
-// each); a piece stores its accumulators here (pf_part_bytes per workgroup).
+// each); a piece stores its accumulators here (pf_part_bytes per piece).
 constexpr int kPfMaxPieces = 4;
-constexpr int pf_part_bytes(int tt) { return kPfBWaves * kPfBRtw * tt * 64 * 16; }
+constexpr int pf_part_bytes(int tt, bool block) { return (block ? kPfBWaves * kPfBRtw : kPfWaves * kPfRtw) * tt * 64 * 16; }
 
 // Rounding forms of the epilogues (FORM, a compile-time set; the ragged kernels use none):
 constexpr int kPfRoundGU = 1;   // gate/up: g and u rounded to bf16 before the SwiGLU (the XLA einsums' bf16 outputs)
@@ -197,7 +197,9 @@ struct PfCb3 {
     };
     static constexpr bool kLdsOnlyBarrier = false;
     static constexpr int kCols = kCb3TileCols;
-    static constexpr bool kSplit = false;   // whole tasks only: K pieces measured slower (561 against 536 us)
+    // the last round's tasks split into K pieces: 71 blocks of the benchmarked layer are 2.2 rounds of workgroups (512
+    // tokens, a few calls in a row 527 -> 466 us; sustained, where the card's power sets the pace, 538 -> 516)
+    static constexpr bool kSplit = true;
     static constexpr int kRtw = kPfRtw, kWaves = kPfWaves;
     static constexpr int kQOff = 4;
     using Wave = Cb3Wave;
@@ -863,7 +865,7 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP, TT> &
             __builtin_amdgcn_make_buffer_rsrc((void *)a.part, (short)0, 0x7fffffff, kBufferWord3);
         const uint32_t lane_off = 16u * (uint32_t)lane;
         auto part_off = [&](int pc, int r, int t) {
-            return (uint32_t)(sti * np + pc) * (uint32_t)pf_part_bytes(TT) +
+            return (uint32_t)(sti * np + pc) * (uint32_t)pf_part_bytes(TT, kBlock) +
                    (uint32_t)((wave * kRtw + r) * TT + t) * 1024u + lane_off;
         };
 #pragma unroll
@@ -968,7 +970,7 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP, TT> &
 }
 
 template <int MODE, class WP, int FORM, int TT>   // MODE 0: gate/up -> h, 1: down -> y; FORM: kPf* rounding forms
-__global__ void __launch_bounds__(64 * WP::kWaves, WP::kCols == 128 ? pf_per_simd(TT) : 2) prefill_kernel(PfArgs a) {
+__global__ void __launch_bounds__(64 * WP::kWaves, pf_per_simd(TT, WP::kCols == 128)) prefill_kernel(PfArgs a) {
     __shared__ PfShared<WP, TT> sh;
     // Workgroups are dispatched to the XCDs round-robin.  The blocks, in launch order (most token tiles first), are
     // dealt to the XCDs eight at a time, all workgroups of a block on one XCD, so the block's activation rows are
