@@ -38,12 +38,28 @@ def _plane_rows(qtype, K):
     raise ValueError(qtype)                     # the reference raises ValueError on an unknown qtype (planes.py:70)
 
 
+# The host side of a call is as long as the smallest calls' GPU work (a router call 18.6 us of Python for 10 us of
+# kernels), so the entry points keep to the cheap forms: the raw handle of the current stream (0.3 us; building
+# torch.cuda.current_stream() 2.8), plain integers for pointers (ctypes converts them by the declared argument types),
+# conversions and slices only where they change something.
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
+
+
+def _as(t, dtype):
+    """t contiguous in dtype (t itself when it is)."""
+    if t.dtype != dtype:
+        t = t.to(dtype)
+    return t if t.is_contiguous() else t.contiguous()
+
+
+def _rows(t, b0, n):
+    """Rows b0 .. b0 + n - 1 of t (t itself when that is all of it; None stays None)."""
+    return t if t is None or (b0 == 0 and n == t.shape[0]) else t[b0:b0 + n]
 
 
 def to_device_planes(planes, device="cuda"):
@@ -201,7 +217,7 @@ class _Workspaces:
 
     def get(self, purpose, nbytes):
         dev = torch.cuda.current_device()
-        key = (dev, torch.cuda.current_stream().cuda_stream, purpose)
+        key = (dev, torch._C._cuda_getCurrentRawStream(dev), purpose)
         buf = self._ws.get(key)
         if buf is None or buf.numel() < nbytes:
             buf = torch.zeros(max(int(nbytes), 256), dtype=torch.uint8, device="cuda")
@@ -341,11 +357,7 @@ def moe_decode(gate, up, down, x, idx, w, limit, shared_expert=-1, want_f32=True
         raise ValueError("f32 activations take the separate launches (phases=3, fused=False)")
     N, k = idx.shape
     x = x.contiguous()
-    if idx.dtype != torch.int32:
-        idx = idx.to(torch.int32)
-    if w.dtype != torch.float32:
-        w = w.to(torch.float32)
-    idx, w = idx.contiguous(), w.contiguous()
+    idx, w = _as(idx, torch.int32), _as(w, torch.float32)
     D = down.rows
     of, ob = out_f32, out_bf16
     if phases & 2:
@@ -383,11 +395,7 @@ def ragged_plan(idx, w, E, tm):
     """ragged_plan (pallas_moe.py:564-592) on the device: idx int32 [T, k], w f32 [T, k] -> dict of device tensors
     blk_expert int32 [G], n_blocks int32 [1], tok_row int32 [Rp], w_row f32 [Rp], row_slot int32 [T, k] with
     G = ceil(T*k / tm) + E, Rp = G * tm (slots sorted stably by expert, every expert padded to whole blocks)."""
-    if idx.dtype != torch.int32:
-        idx = idx.to(torch.int32)
-    if w.dtype != torch.float32:
-        w = w.to(torch.float32)
-    idx, w = idx.contiguous(), w.contiguous()
+    idx, w = _as(idx, torch.int32), _as(w, torch.float32)
     T, k = idx.shape
     G = -(-(T * k) // tm) + E
     dev = idx.device
@@ -425,19 +433,16 @@ def route(x, router_w, bias, k, norm_topk=True, scaling=1.0, workspace=None):
     """The router (moe_route, model.py:798-808) on the device: x bf16 [N, D], router_w f32 [D, E], bias f32 [E] or
     None -> (idx int32 [N, k], w f32 [N, k]).  sigmoid scores, top-k of scores + bias (lower id first on equal
     values), weights = scores (renormalised over the k with ``norm_topk``) times ``scaling``."""
-    if x.dtype != torch.bfloat16:
-        x = x.to(torch.bfloat16)
-    x = x.contiguous()
-    router_w = router_w.to(torch.float32).contiguous()
+    x = _as(x, torch.bfloat16)
+    router_w = _as(router_w, torch.float32)
     if bias is not None:
-        bias = bias.to(torch.float32).contiguous()
+        bias = _as(bias, torch.float32)
     N, D = x.shape
     E = router_w.shape[1]
     if router_w.shape[0] != D or (bias is not None and tuple(bias.shape) != (E,)):
         raise ValueError("route: router_w must be [D, E] = [%d, E] and bias [E]" % D)
-    need = lib().mi_moe_route_workspace(N, D, E)
     if workspace is None:
-        workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+        workspace = WORKSPACES.get("route", lib().mi_moe_route_workspace(N, D, E))
     idx = torch.empty((N, k), dtype=torch.int32, device=x.device)
     w = torch.empty((N, k), dtype=torch.float32, device=x.device)
     check("mi_moe_route", lib().mi_moe_route(_ptr(x), _ptr(router_w), _ptr(bias), N, D, E, int(k),
@@ -482,11 +487,7 @@ def moe_prefill(gate, up, down, x, idx, w, limit, shared_expert=-1, combine="mat
         raise ValueError("chunk must be positive")
     T, k = idx.shape
     x = x.contiguous()
-    if idx.dtype != torch.int32:
-        idx = idx.to(torch.int32)
-    if w.dtype != torch.float32:
-        w = w.to(torch.float32)
-    idx, w = idx.contiguous(), w.contiguous()
+    idx, w = _as(idx, torch.int32), _as(w, torch.float32)
     D = down.rows
     of, ob = out_f32, out_bf16
     if of is None and want_f32:
@@ -635,10 +636,10 @@ def _mlp_many(x, ws3, scales, gu_form, down_form, D, I, limit, yb, yf, workspace
         ws = WORKSPACES.get("mlp_many", need)
     for b0 in range(0, B, _MLP_MANY_STEP):
         n = min(_MLP_MANY_STEP, B - b0)
-        check("mi_mlp_many", lib().mi_mlp_many(_ptr(x[b0:]), n, D, I, _ptr(ws3[0]), _ptr(scales[0]), _ptr(ws3[1]),
+        check("mi_mlp_many", lib().mi_mlp_many(_ptr(_rows(x, b0, n)), n, D, I, _ptr(ws3[0]), _ptr(scales[0]), _ptr(ws3[1]),
                                                _ptr(scales[1]), int(gu_form), _ptr(ws3[2]), _ptr(scales[2]),
-                                               int(down_form), float(limit), _ptr(yb[b0:]),
-                                               _ptr(yf[b0:]) if yf is not None else None, _ptr(ws), ws.numel(),
+                                               int(down_form), float(limit), _ptr(_rows(yb, b0, n)),
+                                               _ptr(_rows(yf, b0, n)), _ptr(ws), ws.numel(),
                                                _stream()))
     return True
 
@@ -671,10 +672,10 @@ def int8_mlp(x, gate, up, down, limit, want_f32=False, y_bf16=None, y_f32=None, 
         if nbytes == 0:
             raise ValueError("mi_int8_mlp: unsupported shape B=%d D=%d I=%d" % (n, D, I))
         ws = workspace if workspace is not None else WORKSPACES.get("int8", nbytes)
-        check("mi_int8_mlp", lib().mi_int8_mlp(_ptr(x[b0:b0 + n]), n, D, I, _ptr(g[0]), _ptr(g[1]), _ptr(u[0]),
+        check("mi_int8_mlp", lib().mi_int8_mlp(_ptr(_rows(x, b0, n)), n, D, I, _ptr(g[0]), _ptr(g[1]), _ptr(u[0]),
                                                _ptr(u[1]), int(g[2]) | gt, _ptr(d[0]), _ptr(d[1]), int(d[2]) | dt,
-                                               float(limit), _ptr(yb[b0:b0 + n]),
-                                               _ptr(yf[b0:b0 + n]) if yf is not None else None, _ptr(ws),
+                                               float(limit), _ptr(_rows(yb, b0, n)),
+                                               _ptr(_rows(yf, b0, n)), _ptr(ws),
                                                ws.numel(), _stream()))
     return (yb, yf) if want_f32 else yb
 
@@ -716,9 +717,9 @@ def bf16_project(x, w, want_f32=False, y_bf16=None, y_f32=None, workspace=None):
         if nbytes == 0:
             raise ValueError("mi_bf16_project: unsupported shape B=%d n_in=%d n_out=%d" % (n, n_in, n_out))
         ws = workspace if workspace is not None else WORKSPACES.get("int8", nbytes)
-        check("mi_bf16_project", lib().mi_bf16_project(_ptr(x[b0:b0 + n]), n, _ptr(wT), n_in, n_out,
-                                                       _ptr(yb[b0:b0 + n]),
-                                                       _ptr(yf[b0:b0 + n]) if yf is not None else None, _ptr(ws),
+        check("mi_bf16_project", lib().mi_bf16_project(_ptr(_rows(x, b0, n)), n, _ptr(wT), n_in, n_out,
+                                                       _ptr(_rows(yb, b0, n)),
+                                                       _ptr(_rows(yf, b0, n)), _ptr(ws),
                                                        ws.numel(), _stream()))
     return (yb, yf) if want_f32 else yb
 
@@ -748,8 +749,8 @@ def bf16_mlp(x, gate, up, down, limit, want_f32=False, y_bf16=None, y_f32=None, 
         if nbytes == 0:
             raise ValueError("mi_bf16_mlp: unsupported shape B=%d D=%d I=%d" % (n, D, I))
         ws = workspace if workspace is not None else WORKSPACES.get("int8", nbytes)
-        check("mi_bf16_mlp", lib().mi_bf16_mlp(_ptr(x[b0:b0 + n]), n, D, I, _ptr(g), _ptr(u), _ptr(d), float(limit),
-                                               _ptr(yb[b0:b0 + n]), _ptr(yf[b0:b0 + n]) if yf is not None else None,
+        check("mi_bf16_mlp", lib().mi_bf16_mlp(_ptr(_rows(x, b0, n)), n, D, I, _ptr(g), _ptr(u), _ptr(d), float(limit),
+                                               _ptr(_rows(yb, b0, n)), _ptr(_rows(yf, b0, n)),
                                                _ptr(ws), ws.numel(), _stream()))
     return (yb, yf) if want_f32 else yb
 
@@ -786,8 +787,9 @@ def decode_chunked(gate, up, down, x, idx, w, limit, shared_expert=-1, out=None)
         out = torch.empty((N, down.rows), dtype=torch.float32, device=x.device)
     for c0 in range(0, N, step):
         c1 = min(N, c0 + step)
-        moe_decode(gate, up, down, x[c0:c1], idx[c0:c1], w[c0:c1], limit, shared_expert=shared_expert,
-                   out_f32=out[c0:c1])
+        n = c1 - c0
+        moe_decode(gate, up, down, _rows(x, c0, n), _rows(idx, c0, n), _rows(w, c0, n), limit,
+                   shared_expert=shared_expert, out_f32=_rows(out, c0, n))
     return out
 
 
