@@ -468,22 +468,39 @@ static size_t i8_lds_bytes(int B, int cols, int scale_axis) {
 // Columns per 2 KB block of a 16-row tile: 128 int8 or 64 bf16 weights.
 static int i8_block_cols(int form) { return form == kW16 ? 64 : 128; }
 
-// Column splits: enough wavefronts to cover the chip (about 3 per SIMD, 3072 over 256 CUs), every wavefront
-// streaming at least 4 blocks (8 KB), the split's staged columns within 48 KB of LDS.  `tiles` counts the 16-row
-// tiles of every projection of the launch.
+// Column splits of a launch; `tiles` counts the 16-row tiles of every projection of it.  Candidates divide the blocks,
+// leave every wavefront at least 4 blocks (8 KB) and stage their columns within 48 KB of LDS.
+//
+// Fewer row groups (4 tiles, a workgroup) than CUs: the weight stream's time at 5 TB/s, stretched by how unevenly the
+// workgroups load the CUs, plus what a split costs (its partials, 4 B bytes per output, and the wait for the last
+// one).  Measured (one launch, us; workgroups per CU in brackets): bf16 6144 -> 4096 1 token S = 4 (1) 14.1, 6 (1.5) 17.0,
+// 12 (3) 15.4; bf16 2048 -> 6144 1 token S = 2 (0.75) 10.3, 8 (3) 9.5, 8 tokens 9.9 and 10.7; bf16 3072 -> 2560 1 token S = 4
+// (0.63) 8.5, 6 (0.94) 7.4, 12 8.4.
+// More row groups: about 3 wavefronts per SIMD (3072 over 256 CUs) in flight.
 static int i8_splits(int B, int n_in, int tiles, int scale_axis) {
     const int nblk = n_in / i8_block_cols(scale_axis);
     const int forced = tuning(kTuneI8S, 0);       // measurements: a forced split count (must divide the blocks)
     if (forced > 0 && nblk % forced == 0 && i8_lds_bytes(B, n_in / forced, scale_axis) <= 48 * 1024) return forced;
-    int target = tuning(kTuneI8Waves, 3072);       // wavefronts to aim for
-    if (target <= 0) target = 3072;
+    const int waves = tuning(kTuneI8Waves, 0);     // measurements: wavefronts to aim for
+    constexpr int kCus = 256;
+    const int groups = (tiles + kI8Waves - 1) / kI8Waves;
+    const bool few = groups < kCus && waves <= 0;
+    const double stream = (double)tiles * 16 * n_in * (scale_axis == kW16 ? 2 : 1) / 5e6;      // us
+    const int target = waves > 0 ? waves : 3072;
     int best = 1;
+    double best_us = 1e30;
     for (int S = 1; S <= nblk; ++S) {
         if (nblk % S) continue;
         if (i8_lds_bytes(B, n_in / S, scale_axis) > 48 * 1024) continue;
         if (nblk / S < 4 && S > 1) break;
-        best = S;
-        if ((long long)tiles * S >= target) break;
+        if (few) {
+            const int wgs = groups * S, rounds = (wgs + kCus - 1) / kCus;
+            const double us = stream * rounds * kCus / wgs + S * (0.12 + 0.03 * B);
+            if (us < best_us) best_us = us, best = S;
+        } else {
+            best = S;
+            if ((long long)tiles * S >= target) break;
+        }
     }
     return best;
 }
