@@ -47,7 +47,7 @@ EXPORTS = ("mi_matvec", "mi_matvec_workspace", "mi_moe_decode", "mi_moe_decode_f
            "mi_ragged_plan", "mi_moe_prefill", "mi_moe_prefill_workspace", "mi_moe_prefill_form",
            "mi_moe_prefill_form_workspace", "mi_dequant", "mi_int8_project", "mi_int8_project_workspace", "mi_int8_project_many",
            "mi_int8_project_many_workspace", "mi_int8_mlp", "mi_int8_mlp_workspace", "mi_moe_route", "mi_moe_route_workspace", "mi_pack_planes", "mi_int8_tile", "mi_bf16_project", "mi_bf16_project_workspace",
-           "mi_bf16_mlp", "mi_bf16_mlp_workspace", "mi_tuning_set", "mi_tuning_reset",
+           "mi_bf16_mlp", "mi_mlp_many", "mi_mlp_many_workspace", "mi_bf16_mlp_workspace", "mi_tuning_set", "mi_tuning_reset",
            "mi_strerror",
            "mi_version")
 

@@ -1,0 +1,24 @@
+"""CPU: host validation of mi_mlp_many (no launch: every call here is refused) and the sizes its workspace function
+takes and refuses."""
+import ctypes
+
+
+def test_mlp_many_validation(pkg):
+    L, lib = pkg._lib.lib(), pkg._lib
+    P = ctypes.c_void_p
+
+    def call(B=64, D=512, I=256, gf=lib.MI_I8_COL_SCALES, df=lib.MI_I8_COL_SCALES, gw=P(0x1000), gs=P(0x2000), limit=7.0,
+             x=P(0x10000), y=P(0x20000), wsb=1 << 30):
+        return L.mi_mlp_many(x, B, D, I, gw, gs, P(0x3000), P(0x4000), gf, P(0x5000), P(0x6000), df, ctypes.c_float(limit),
+                             y, None, P(0x100000), wsb, None)
+
+    assert call(B=0) == 4 and call(B=(1 << 14) + 1) == 4                                # MI_ERR_TOKENS
+    assert call(D=640) == 3 and call(I=300) == 3                                        # MI_ERR_SHAPE
+    assert call(limit=0.0) == 8 and call(gw=P(0x1008)) == 8 and call(x=P(0x10002)) == 8  # MI_ERR_ARG
+    assert call(gf=lib.MI_I8_COL_AFTER) == 8 and call(gf=lib.MI_W_BF16 | lib.MI_I8_TILED) == 8
+    assert call(gf=lib.MI_I8_ROW_SCALES, gs=P(0x2004)) == 8
+    assert call(gw=None) == 1 and call(gs=None) == 1 and call(y=None) == 1              # MI_ERR_NULL
+    assert call(wsb=16) == 5                                                            # MI_ERR_WORKSPACE
+    assert L.mi_mlp_many_workspace(512, 6144, 2048) > 0
+    for bad in ((0, 512, 256), (64, 500, 256), (64, 512, 100), (64, 131072, 256), (64, 65536, 32768)):
+        assert L.mi_mlp_many_workspace(*bad) == 0, bad
