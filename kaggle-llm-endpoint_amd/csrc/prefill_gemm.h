@@ -3,8 +3,9 @@
 // prefill branches, resident.py:122-135,169-210):
 //   prefill_kernel<MODE, WP, FORM>  one workgroup per (block, row range) streams the block's expert once for all
 //                       its rows: each wavefront owns 64 (CB3) or 32 weight rows x up to 80 rows of activations (5
-//                       MFMA token tiles), decodes every weight once (CB3: the decoder of cb3_tiles.h; IQ3_S: the planes straight
-//                       into the A operand) and reuses it across the token tiles; the block's activation rows are
+//                       MFMA token tiles; 128 and 8 in the wide launches), decodes every weight once (CB3: the decoder
+//                       of cb3_tiles.h; the block formats: the planes straight into the A operand) and reuses it
+//                       across the token tiles; the block's activation rows are
 //                       staged one column tile (160 / 128 columns) at a time in LDS;
 //                         gate/up: h = bf16(silu(min(g, L)) * clip(u, -L, L)), g and u f32    (pallas_moe.py:682)
 //                         down:    y = bf16(h Wd^T), f32 accumulation                        (pallas_moe.py:747)
