@@ -31,7 +31,7 @@ struct PlanOut {
     float *w_row;          // [Rp]  routing weight of every sorted row, 0 = padding
     int32_t *row_slot;     // [T * kk] sorted row of every (token, slot); -1 for an expert id outside [0, E)
     int32_t *blk_n;        // [G]   rows of every block that are not padding (NULL: not written)
-    int32_t *blk_order;    // [G]   blocks in launch order: most token tiles first (NULL: not written)
+    int32_t *blk_order;    // [G]   blocks in launch order: most token tiles first, then by index (NULL: not written)
     int even;              // an expert's blocks share its rows evenly, in multiples of 16 (0: whole blocks of tm first)
     int merge_dups;        // w_row of the first slot of a token's expert = the sum of that token's weights of the
                            // expert in column order, 0 for its later slots (the sweeps' summed routing weight)
@@ -107,7 +107,8 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
     __shared__ unsigned long long lanes[kPlanWaves][kPlanMaskE];   // pass 2: lanes of every id in this step
     __shared__ int wsum[kPlanWaves];
     __shared__ int per[kPlanMaxE];                // rows per block of every expert (the last one fewer)
-    __shared__ int ntile[kPfWideTT + 1];           // blocks of every token tile count, then the first position of each
+    __shared__ int ntile[kPfWideTT + 1];           // blocks of every token tile count, then the next position of each
+    __shared__ int wtile[kPlanWaves][kPfWideTT + 1];   // blocks of every token tile count per wavefront
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kk = k + (shared >= 0 ? 1 : 0);
     const int S = T * kk;
@@ -268,9 +269,9 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
         if (p.blk_order && n > 0) atomicAdd(&ntile[(n + 15) >> 4], 1);
     }
     if (!p.blk_order) return;
-    // launch order: a counting sort by token tiles, most first, so the launches' last tasks are their shortest (the
-    // order among equals is free: it changes no result)
-    vm_wait<0>();                                 // blk_n as stored above
+    // launch order: a stable counting sort by token tiles, most first, so the launches' last tasks are their shortest.
+    // Equal blocks stay in block order: the GEMMs split the last blocks of this order along K, another f32 summation
+    // order, so which blocks those are must not depend on which wavefront comes first.
     __syncthreads();
     if (tid == 0) {
         int at = 0;
@@ -281,7 +282,27 @@ __global__ void __launch_bounds__(kPlanThreads) ragged_plan_kernel(const int32_t
         }
     }
     __syncthreads();
-    for (int g = tid; g < n_blocks; g += kPlanThreads) p.blk_order[atomicAdd(&ntile[(p.blk_n[g] + 15) >> 4], 1)] = g;
+    for (int g0 = 0; g0 < n_blocks; g0 += kPlanThreads) {
+        const int g = g0 + tid;
+        const int c = g < n_blocks ? (p.blk_n[g] + 15) >> 4 : 0;      // blk_n[g]: this thread's own store above
+        int below = 0;                                                // lower lanes of the same count
+        for (int v = 1; v <= kPfWideTT; ++v) {
+            const uint64_t m = __ballot(c == v);
+            if (c == v) below = __popcll(m & ((1ull << lane) - 1ull));
+            if (lane == 0) wtile[wave][v] = __popcll(m);
+        }
+        __syncthreads();
+        if (c) {
+            int at = ntile[c] + below;
+            for (int v = 0; v < wave; ++v) at += wtile[v][c];
+            p.blk_order[at] = g;
+        }
+        if (g0 + kPlanThreads >= n_blocks) break;
+        __syncthreads();
+        if (tid > 0 && tid <= kPfWideTT)
+            for (int v = 0; v < kPlanWaves; ++v) ntile[tid] += wtile[v][tid];
+        __syncthreads();
+    }
 }
 
 // out[t] = sum_j wt(t, j) * y[row_slot(t, j)] over the plan's kk columns in order, f32; wt = bf16(w) for the matmul
