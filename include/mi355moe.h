@@ -394,8 +394,8 @@ size_t mi_bf16_mlp_workspace(int32_t B, int32_t D, int32_t I);
  * mlp_partial for many tokens (a prompt piece; 1 <= B <= 16384): the steps, shapes, weight layouts and rounding points
  * of mi_int8_mlp and mi_bf16_mlp, as dense GEMMs that meet a weight tile with up to 128 tokens.  gu_form / down_form:
  * MI_I8_ROW_SCALES or MI_I8_COL_SCALES (| MI_I8_TILED) over int8, or MI_W_BF16.  x, the weights, y_f32, the workspace
- * and per-row scales 16-byte aligned, y_bf16 8-byte.  Workspace: mi_mlp_many_workspace bytes, no counters: its
- * contents need no initialisation.
+ * and per-row scales 16-byte aligned, y_bf16 8-byte.  Workspace: mi_mlp_many_workspace bytes (enough for every smaller
+ * B of the same D and I too), no counters: its contents need no initialisation.
  */
 int mi_mlp_many(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I, const void *gate_w, const float *gate_s,
                 const void *up_w, const float *up_s, int32_t gu_form, const void *down_w, const float *down_s,

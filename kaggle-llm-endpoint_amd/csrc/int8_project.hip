@@ -717,9 +717,16 @@ static bool dg_layout(int B, int D, int I, DgLayout &L) {
 
 extern "C" {
 
+// Never less than a call of fewer tokens needs (few tokens are split into more partials), so that a workspace sized for
+// a caller's largest piece serves every piece.  dg_plan is the same within each 64 tokens, where the size grows with B.
 size_t mi_mlp_many_workspace(int32_t B, int32_t D, int32_t I) {
     DgLayout L;
-    return dg_layout(B, D, I, L) ? L.total : 0;
+    size_t need = 0;
+    for (int b = 0; b < B; b += 64) {
+        if (!dg_layout(std::min(b + 64, B), D, I, L)) return 0;
+        need = std::max(need, L.total);
+    }
+    return need;
 }
 
 int mi_mlp_many(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I, const void *gate_w, const float *gate_s,

@@ -66,3 +66,22 @@ def test_mlp_many_other_routes(pkg, gpu):
         yf = pkg.int8_mlp(xt, *leaves, 7.0, want_f32=True, workspace=ws)[1]
         assert rel_l2(yf.cpu().numpy(), want) < 1e-4
         assert int(ws[:pkg._lib.I8_CTR_BYTES].count_nonzero()) == 0
+
+
+def test_mlp_many_last_piece(pkg, gpu):
+    """More than the 4096 tokens of one piece, the last piece of a size whose split sums need more scratch than the
+    first's: the bits of the pieces by themselves, without and with a kept workspace sized for the first piece."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(11)
+    B, D, I = 4096 + 512, 2048, 768
+    w = [torch.randn(s, device="cuda", generator=gen).to(torch.bfloat16) * 0.02 for s in ((D, I), (D, I), (I, D))]
+    leaves = [pkg.bf16_leaf(v) for v in w]
+    x = torch.randn((B, D), device="cuda", generator=gen).to(torch.bfloat16)
+    kept = torch.zeros(pkg._lib.I8_CTR_BYTES + pkg._lib.lib().mi_mlp_many_workspace(4096, D, I), dtype=torch.uint8,
+                       device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        got = [pkg.bf16_mlp(x, *leaves, 7.0, workspace=ws) for ws in (None, kept)]
+        want = torch.cat([pkg.bf16_mlp(x[:4096], *leaves, 7.0), pkg.bf16_mlp(x[4096:], *leaves, 7.0)])
+        torch.cuda.synchronize()
+    assert torch.equal(got[0], want) and torch.equal(got[1], want)

@@ -22,3 +22,12 @@ def test_mlp_many_validation(pkg):
     assert L.mi_mlp_many_workspace(512, 6144, 2048) > 0
     for bad in ((0, 512, 256), (64, 500, 256), (64, 512, 100), (64, 131072, 256), (64, 65536, 32768)):
         assert L.mi_mlp_many_workspace(*bad) == 0, bad
+
+
+def test_mlp_many_workspace_serves_fewer_tokens(pkg):
+    """A call of more than 4096 tokens runs 4096 at a time and its last piece in the same workspace: no piece needs
+    more than the size of the largest."""
+    size = pkg._lib.lib().mi_mlp_many_workspace
+    for D, I in ((6144, 2048), (4096, 1536), (3072, 1280), (2048, 768), (256, 256), (65536, 256)):
+        sizes = [size(b, D, I) for b in range(1, 4097)]
+        assert all(a <= b for a, b in zip(sizes, sizes[1:])), (D, I)
