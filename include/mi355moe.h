@@ -315,6 +315,7 @@ int mi_dequant(const mi_table *t, int32_t expert, float *out, void *stream);
  * every int8 call leaves them zero, so mi_int8_project, mi_int8_project_many and mi_int8_mlp may share one
  * workspace, ordered on one stream.  One launch: the workgroup that completes a row group's splits last adds the
  * partials in split order (a second, summing launch when a launch has more than 1024 row groups of 64 outputs).
+ * The int8 and bf16 projection and MLP workspace sizes serve every smaller B of the same shape too.
  * scale_axis | MI_I8_TILED: qT is in the tiled layout that mi_int8_tile writes (same values, another byte order).
  */
 #define MI_I8_ROW_SCALES 0

@@ -477,32 +477,50 @@ static int i8_block_cols(int form) { return form == kW16 ? 64 : 128; }
 // 12 (3) 15.4; bf16 2048 -> 6144 1 token S = 2 (0.75) 10.3, 8 (3) 9.5, 8 tokens 9.9 and 10.7; bf16 3072 -> 2560 1 token S = 4
 // (0.63) 8.5, 6 (0.94) 7.4, 12 8.4.
 // More row groups: about 3 wavefronts per SIMD (3072 over 256 CUs) in flight.
-static int i8_splits(int B, int n_in, int tiles, int scale_axis) {
+//
+// Writes S[b - b0] for every token count b of b0 .. b1 (up to 32 of them).
+static void i8_splits_of(int b0, int b1, int n_in, int tiles, int scale_axis, int *S) {
     const int nblk = n_in / i8_block_cols(scale_axis);
     const int forced = tuning(kTuneI8S, 0);       // measurements: a forced split count (must divide the blocks)
-    if (forced > 0 && nblk % forced == 0 && i8_lds_bytes(B, n_in / forced, scale_axis) <= 48 * 1024) return forced;
     const int waves = tuning(kTuneI8Waves, 0);     // measurements: wavefronts to aim for
     constexpr int kCus = 256;
     const int groups = (tiles + kI8Waves - 1) / kI8Waves;
     const bool few = groups < kCus && waves <= 0;
     const double stream = (double)tiles * 16 * n_in * (scale_axis == kW16 ? 2 : 1) / 5e6;      // us
     const int target = waves > 0 ? waves : 3072;
-    int best = 1;
-    double best_us = 1e30;
-    for (int S = 1; S <= nblk; ++S) {
-        if (nblk % S) continue;
-        if (i8_lds_bytes(B, n_in / S, scale_axis) > 48 * 1024) continue;
-        if (nblk / S < 4 && S > 1) break;
-        if (few) {
-            const int wgs = groups * S, rounds = (wgs + kCus - 1) / kCus;
-            const double us = stream * rounds * kCus / wgs + S * (0.12 + 0.03 * B);
-            if (us < best_us) best_us = us, best = S;
-        } else {
-            best = S;
-            if ((long long)tiles * S >= target) break;
+    double best_us[32];
+    bool done[32];
+    for (int b = b0; b <= b1; ++b) {
+        S[b - b0] = 1;
+        best_us[b - b0] = 1e30;
+        done[b - b0] = false;
+        if (forced > 0 && nblk % forced == 0 && i8_lds_bytes(b, n_in / forced, scale_axis) <= 48 * 1024) {
+            S[b - b0] = forced;
+            done[b - b0] = true;
         }
     }
-    return best;
+    for (int c = 1; c <= nblk && (c == 1 || nblk / c >= 4); ++c) {
+        if (nblk % c) continue;
+        const int wgs = groups * c, rounds = (wgs + kCus - 1) / kCus;
+        const double us = stream * rounds * kCus / wgs;
+        for (int b = b0; b <= b1; ++b) {
+            const int i = b - b0;
+            if (done[i] || i8_lds_bytes(b, n_in / c, scale_axis) > 48 * 1024) continue;
+            if (few) {
+                const double v = us + c * (0.12 + 0.03 * b);
+                if (v < best_us[i]) best_us[i] = v, S[i] = c;
+            } else {
+                S[i] = c;
+                done[i] = (long long)tiles * c >= target;
+            }
+        }
+    }
+}
+
+static int i8_splits(int B, int n_in, int tiles, int scale_axis) {
+    int S;
+    i8_splits_of(B, B, n_in, tiles, scale_axis, &S);
+    return S;
 }
 
 static int i8_tiles(const int32_t *n_out, int n_proj) {
@@ -511,14 +529,19 @@ static int i8_tiles(const int32_t *n_out, int n_proj) {
     return t;
 }
 
-// Partial bytes of one launch: the f32 split partials (none with one split, except for an MLP's gate/up pair,
-// whose SwiGLU reads them).
-static size_t i8_part_bytes(int B, int n_in, const int32_t *n_out, int n_proj, int scale_axis, int pair) {
+// Partial bytes of one launch of B tokens: the f32 split partials (none with one split, except for an MLP's gate/up
+// pair, whose SwiGLU reads them).  upto: the largest of these over 1 .. B tokens (fewer tokens can have more splits), so
+// that a workspace sized for a caller's largest batch serves every batch.
+static size_t i8_part_bytes(int B, int n_in, const int32_t *n_out, int n_proj, int scale_axis, int pair, bool upto) {
     scale_axis &= ~MI_I8_TILED;
-    size_t total = 0;
+    size_t total = 0, need = 0;
     for (int j = 0; j < n_proj; ++j) total += (size_t)n_out[j];
-    const int S = i8_splits(B, n_in, i8_tiles(n_out, n_proj), scale_axis);
-    return S == 1 && !pair ? 256 : sizeof(float) * (size_t)S * B * total;
+    int S[32];
+    const int b0 = upto ? 1 : B;
+    i8_splits_of(b0, B, n_in, i8_tiles(n_out, n_proj), scale_axis, S);
+    for (int b = b0; b <= B; ++b)
+        need = std::max(need, S[b - b0] == 1 && !pair ? 256 : sizeof(float) * (size_t)S[b - b0] * b * total);
+    return need;
 }
 
 static size_t al256_i8(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -551,7 +574,7 @@ static int i8_launch(const uint16_t *x_bf16, int32_t B, int32_t n_in, const mi_i
         if (p.n_out <= 0 || p.n_out % 16) return MI_ERR_SHAPE;
         n_out[j] = p.n_out;
     }
-    const size_t need = i8_part_bytes(B, n_in, n_out, n_proj, scale_axis, pair);
+    const size_t need = i8_part_bytes(B, n_in, n_out, n_proj, scale_axis, pair, false);
     if (!part || part_bytes < need || (uintptr_t)part % 16) return MI_ERR_WORKSPACE;
     I8Args a{};
     a.pair = pair;
@@ -617,11 +640,11 @@ static int i8_launch(const uint16_t *x_bf16, int32_t B, int32_t n_in, const mi_i
 // mlp_partial's two launches over weights of one form per launch (int8 with scales, or kW16): gate and up together
 // (their last workgroups form h), then down with its split sums.  Workspace: [counter blocks: gate/up's, down's]
 // [gate/up partials][h][down partials].
-static size_t mlp_workspace(int32_t B, int32_t D, int32_t I, int32_t gu_form, int32_t dn_form) {
+static size_t mlp_workspace(int32_t B, int32_t D, int32_t I, int32_t gu_form, int32_t dn_form, bool upto) {
     if (B <= 0 || B > 32 || D <= 0 || I <= 0 || D % 256 || I % 256) return 0;
     const int32_t gu[2] = {I, I}, dn = D;
-    return kI8CtrBytes + al256_i8(i8_part_bytes(B, D, gu, 2, gu_form, 1)) + al256_i8(2 * (size_t)B * I) +
-           i8_part_bytes(B, I, &dn, 1, dn_form, 0);
+    return kI8CtrBytes + al256_i8(i8_part_bytes(B, D, gu, 2, gu_form, 1, upto)) + al256_i8(2 * (size_t)B * I) +
+           i8_part_bytes(B, I, &dn, 1, dn_form, 0, upto);
 }
 
 static int mlp_launches(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I, const int8_t *gate_w,
@@ -629,13 +652,13 @@ static int mlp_launches(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I,
                         const int8_t *down_w, const float *down_s, int32_t dn_form, float limit, uint16_t *y_bf16,
                         float *y_f32, void *workspace, size_t workspace_bytes, void *stream) {
     if (!(limit > 0.0f)) return MI_ERR_ARG;
-    const size_t need = mlp_workspace(B, D, I, gu_form & ~MI_I8_TILED, dn_form & ~MI_I8_TILED);
+    const size_t need = mlp_workspace(B, D, I, gu_form & ~MI_I8_TILED, dn_form & ~MI_I8_TILED, false);
     if (need == 0) return MI_ERR_ARG;
     if (!workspace || workspace_bytes < need || (uintptr_t)workspace % 256) return MI_ERR_WORKSPACE;
     const int32_t gu[2] = {I, I};
     uint32_t *cnt = (uint32_t *)workspace;
     char *gu_part = (char *)workspace + kI8CtrBytes;
-    const size_t part = al256_i8(i8_part_bytes(B, D, gu, 2, gu_form, 1));
+    const size_t part = al256_i8(i8_part_bytes(B, D, gu, 2, gu_form, 1, false));
     uint16_t *h = (uint16_t *)(gu_part + part);
     char *dn_part = gu_part + part + al256_i8(2 * (size_t)B * I);
     const mi_i8_proj p[2] = {{gate_w, gate_s, I, nullptr, nullptr}, {up_w, up_s, I, nullptr, nullptr}};
@@ -817,7 +840,7 @@ size_t mi_int8_project_many_workspace(int32_t B, int32_t n_in, const int32_t *n_
     if (scale_axis < MI_I8_ROW_SCALES || scale_axis > MI_I8_COL_AFTER) return 0;
     for (int j = 0; j < n_proj; ++j)
         if (n_out[j] <= 0 || n_out[j] % 16) return 0;
-    return kI8CtrBytes + i8_part_bytes(B, n_in, n_out, n_proj, scale_axis, 0);
+    return kI8CtrBytes + i8_part_bytes(B, n_in, n_out, n_proj, scale_axis, 0, true);
 }
 
 // Every int8 workspace starts with the counter blocks (kI8CtrBytes), then the launch's data.
@@ -859,7 +882,7 @@ size_t mi_int8_mlp_workspace(int32_t B, int32_t D, int32_t I, int32_t gu_scale_a
     down_scale_axis &= ~MI_I8_TILED;
     if (gu_scale_axis != MI_I8_ROW_SCALES && gu_scale_axis != MI_I8_COL_SCALES) return 0;
     if (down_scale_axis != MI_I8_ROW_SCALES && down_scale_axis != MI_I8_COL_SCALES) return 0;
-    return mlp_workspace(B, D, I, gu_scale_axis, down_scale_axis);
+    return mlp_workspace(B, D, I, gu_scale_axis, down_scale_axis, true);
 }
 
 int mi_int8_mlp(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I, const int8_t *gate_qT, const float *gate_s,
@@ -870,14 +893,14 @@ int mi_int8_mlp(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I, const i
         return MI_ERR_NULL;
     if (B <= 0 || B > 32) return MI_ERR_TOKENS;
     if (D <= 0 || I <= 0 || D % 256 || I % 256) return MI_ERR_SHAPE;
-    if (mi_int8_mlp_workspace(B, D, I, gu_scale_axis, down_scale_axis) == 0) return MI_ERR_ARG;
+    if (mi_int8_mlp_workspace(1, D, I, gu_scale_axis, down_scale_axis) == 0) return MI_ERR_ARG;      // scale forms
     return mlp_launches(x_bf16, B, D, I, gate_qT, gate_s, up_qT, up_s, gu_scale_axis, down_qT, down_s,
                         down_scale_axis, limit, y_bf16, y_f32, workspace, workspace_bytes, stream);
 }
 
 size_t mi_bf16_project_workspace(int32_t B, int32_t n_in, int32_t n_out) {
     if (B <= 0 || B > 32 || n_in <= 0 || n_in % 256 || n_out <= 0 || n_out % 16) return 0;
-    return kI8CtrBytes + i8_part_bytes(B, n_in, &n_out, 1, kW16, 0);
+    return kI8CtrBytes + i8_part_bytes(B, n_in, &n_out, 1, kW16, 0, true);
 }
 
 int mi_bf16_project(const uint16_t *x_bf16, int32_t B, const uint16_t *wT, int32_t n_in, int32_t n_out,
@@ -892,7 +915,7 @@ int mi_bf16_project(const uint16_t *x_bf16, int32_t B, const uint16_t *wT, int32
                      ok ? workspace_bytes - kI8CtrBytes : 0, (uint32_t *)workspace, stream, 0, 0.0f, nullptr);
 }
 
-size_t mi_bf16_mlp_workspace(int32_t B, int32_t D, int32_t I) { return mlp_workspace(B, D, I, kW16, kW16); }
+size_t mi_bf16_mlp_workspace(int32_t B, int32_t D, int32_t I) { return mlp_workspace(B, D, I, kW16, kW16, true); }
 
 int mi_bf16_mlp(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I, const uint16_t *gate_wT,
                 const uint16_t *up_wT, const uint16_t *down_wT, float limit, uint16_t *y_bf16, float *y_f32,
