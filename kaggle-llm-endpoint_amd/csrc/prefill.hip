@@ -586,7 +586,7 @@ static bool pf_bytes_ok(long long T, long long kk, long long E, long long I, lon
 // (250) 1996 / 1734; Q2_K + Q3_K the same way.
 static int pf_tt(const mi_table *gate, const mi_table *down, int T, int kk) {
     const int E = gate->n_experts;
-    if (gate->qtype == MI_QT_CB3 || down->qtype == MI_QT_CB3) return kPfTT;
+    if (E <= 0 || gate->qtype == MI_QT_CB3 || down->qtype == MI_QT_CB3) return kPfTT;      // E <= 0: refused by the caller
     const long long S = (long long)T * kk;
     const auto blocks = [&](long long tm) { return (S + tm * E - 1) / (tm * E); };      // of an expert of S / E rows
     if (!tuning(kTunePfWide, blocks(16 * kPfWideTT) < blocks(16 * kPfTT))) return kPfTT;
