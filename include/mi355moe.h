@@ -252,7 +252,8 @@ int mi_ragged_plan(const int32_t *idx, const float *w, int32_t T, int32_t k, int
  * Every expert's weights are read once per block of 80 rows. T*(k+1) <= 2^22, E <= 1024, gate.rows % 128 == 0,
  * down.rows % 256 == 0; the IQ formats also need cols % 256 == 0. MI_ERR_MISMATCH when gate and up differ in format
  * or shape. Four launches: plan, gate/up, down, combine. The workspace (mi_moe_prefill_workspace bytes) holds the
- * plan, h and y; it needs no initialisation.
+ * plan, h and y; it needs no initialisation.  The workspace sizes of the prefill serve every smaller T of the same tables,
+ * k, shared_expert and combine too.
  */
 #define MI_COMBINE_MATMUL 0
 #define MI_COMBINE_GATHER 1

@@ -584,14 +584,34 @@ static bool pf_bytes_ok(long long T, long long kk, long long E, long long I, lon
 // With the same number the narrow launches' third wavefront per SIMD wins.  D 6144, I 2048, 64 experts, top-8, narrow /
 // wide: IQ3_S 512 tokens (64 rows) 599 / 635 us, 700 (88) 889 / 721, 900 (113) 1033 / 852, 1200 (150) 1247 / 1303, 1999
 // (250) 1996 / 1734; Q2_K + Q3_K the same way.
-static int pf_tt(const mi_table *gate, const mi_table *down, int T, int kk) {
-    const int E = gate->n_experts;
-    if (E <= 0 || gate->qtype == MI_QT_CB3 || down->qtype == MI_QT_CB3) return kPfTT;      // E <= 0: refused by the caller
-    const long long S = (long long)T * kk;
+static bool pf_prefers_wide(const mi_table *gate, const mi_table *down, long long T, int kk) {
+    const long long S = T * kk, E = gate->n_experts;
+    if (E <= 0 || gate->qtype == MI_QT_CB3 || down->qtype == MI_QT_CB3) return false;      // E <= 0: refused by the caller
     const auto blocks = [&](long long tm) { return (S + tm * E - 1) / (tm * E); };      // of an expert of S / E rows
-    if (!tuning(kTunePfWide, blocks(16 * kPfWideTT) < blocks(16 * kPfTT))) return kPfTT;
-    return plan_sizes_ok(T, kk, E, 16 * kPfWideTT) && pf_bytes_ok(T, kk, E, gate->rows, down->rows, kPfWideTT) ? kPfWideTT
-                                                                                                             : kPfTT;
+    return tuning(kTunePfWide, blocks(16 * kPfWideTT) < blocks(16 * kPfTT)) != 0;
+}
+
+static bool pf_sizes_ok(const mi_table *gate, const mi_table *down, long long T, int kk, int tt) {
+    return plan_sizes_ok(T, kk, gate->n_experts, 16 * tt) &&
+           pf_bytes_ok(T, kk, gate->n_experts, gate->rows, down->rows, tt);
+}
+
+static int pf_tt(const mi_table *gate, const mi_table *down, int T, int kk) {
+    return pf_prefers_wide(gate, down, T, kk) && pf_sizes_ok(gate, down, T, kk, kPfWideTT) ? kPfWideTT : kPfTT;
+}
+
+// The largest token count up to T whose plan is wide (0: none).  Plans are wide from 80 to 128 rows per expert and again
+// above 160, as far as their buffers' offsets fit.
+static int pf_last_wide(const mi_table *gate, const mi_table *down, int T, int kk) {
+    int lo = 0, hi = T;                                 // the largest count whose wide plan fits
+    while (lo < hi) {
+        const int mid = lo + (hi - lo + 1) / 2;
+        if (pf_sizes_ok(gate, down, mid, kk, kPfWideTT)) lo = mid;
+        else hi = mid - 1;
+    }
+    if (lo > 0 && pf_prefers_wide(gate, down, lo, kk)) return lo;
+    const int t1 = (int)std::min<long long>(lo, 16ll * kPfWideTT * gate->n_experts / kk);      // 128 rows per expert
+    return t1 > 0 && pf_prefers_wide(gate, down, t1, kk) ? t1 : 0;
 }
 
 static int launch_plan(const int32_t *idx, const float *w, int T, int k, int shared, int E, int tm, PlanOut p,
@@ -621,9 +641,14 @@ size_t mi_moe_prefill_form_workspace(const mi_table *gate, const mi_table *down,
                                      int32_t shared_expert, int32_t combine) {
     if (!gate || !down || k <= 0 || combine < MI_COMBINE_MATMUL || combine > MI_COMBINE_XLA_SWEEP) return 0;
     const int kk = k + (shared_expert >= 0 ? 1 : 0);
-    const int E = gate->n_experts, tt = pf_tt(gate, down, T, kk);
-    if (!plan_sizes_ok(T, kk, E, 16 * tt) || !pf_bytes_ok(T, kk, E, gate->rows, down->rows, tt)) return 0;
-    return pf_layout(T, kk, E, gate->rows, down->rows, pf_y32(combine), tt).total;
+    if (T <= 0 || !pf_sizes_ok(gate, down, T, kk, pf_tt(gate, down, T, kk))) return 0;
+    // Never less than a call of fewer tokens needs, so that a workspace sized for a caller's longest piece serves every
+    // piece: a wide plan pads an expert's rows to more than a narrow plan of more tokens does.
+    const auto size = [&](int t, int tt) {
+        return pf_layout(t, kk, gate->n_experts, gate->rows, down->rows, pf_y32(combine), tt).total;
+    };
+    const int tw = pf_last_wide(gate, down, T, kk);
+    return tw ? std::max(size(T, kPfTT), size(tw, kPfWideTT)) : size(T, kPfTT);
 }
 
 size_t mi_moe_prefill_workspace(const mi_table *gate, const mi_table *down, int32_t T, int32_t k,
@@ -653,7 +678,7 @@ int mi_moe_prefill_form(const mi_table *gate, const mi_table *up, const mi_table
     if (shared_expert >= E || shared_expert < -1) return MI_ERR_ARG;
     const int kk = k + (shared_expert >= 0 ? 1 : 0);
     const int tt = pf_tt(gate, down, T, kk);
-    if (!plan_sizes_ok(T, kk, E, 16 * tt) || !pf_bytes_ok(T, kk, E, I, D, tt)) return MI_ERR_TOKENS;
+    if (!pf_sizes_ok(gate, down, T, kk, tt)) return MI_ERR_TOKENS;
     if (!(limit > 0.0f) || combine < MI_COMBINE_MATMUL || combine > MI_COMBINE_XLA_SWEEP) return MI_ERR_ARG;
     if (combine == MI_COMBINE_XLA_SWEEP && chunk <= 0) return MI_ERR_ARG;
     const bool y32 = pf_y32(combine);
