@@ -466,10 +466,14 @@ static PfLayout pf_layout(int T, int kk, int E, int I, int D, bool y32, int tt) 
     L.off_rs = o; o = al256(o + 4 * (size_t)L.S);
     L.off_h = o; o = al256(o + 2 * (size_t)L.Rp * I);
     L.off_y = o; o = al256(o + (y32 ? 4 : 2) * (size_t)L.Rp * D);
-    // either GEMM may be of a block format or CB3
-    L.P = std::max(pf_slots(tt, true), pf_slots(tt, false));
-    L.off_part = o; o = al256(o + std::max((size_t)pf_slots(tt, true) * pf_part_bytes(tt, true),
-                                           (size_t)pf_slots(tt, false) * pf_part_bytes(tt, false)));
+    // either GEMM may be of a block format or, in narrow plans, CB3
+    size_t part = 0;
+    for (const bool block : {true, false}) {
+        if (!block && tt > kPfTT) continue;
+        L.P = std::max(L.P, pf_slots(tt, block));
+        part = std::max(part, (size_t)pf_slots(tt, block) * pf_part_bytes(tt, block));
+    }
+    L.off_part = o; o = al256(o + part);
     L.off_cnt = o; o = al256(o + 4 * (size_t)L.P);
     L.total = o;
     return L;

@@ -35,3 +35,14 @@ def test_sizes_grow_with_the_piece(pkg, gate, down, E, k, shared, combine):
     assert len(sizes) > 50 and all(n > 0 for _, n in sizes)
     for (t0, a), (t1, b) in zip(sizes, sizes[1:]):
         assert a <= b, (t0, a, t1, b)
+
+
+@pytest.mark.parametrize("T,tm", [(512, 80), (1024, 128), (1999, 128)])
+def test_size_is_rows_and_piece_sums(pkg, T, tm):
+    """The padded rows of h and y, the plan's arrays and the split tasks' piece sums: 40 KB on each of 3 slots per CU or
+    80 KB (CB3) on 2 in narrow plans, 64 KB on 2 in wide ones; 256 CUs."""
+    L, E, k, I, D = pkg._lib.lib(), 64, 8, 2048, 6144
+    G = -(-T * k // tm) + E
+    need = G * tm * 2 * (I + D) + 4 * (3 * G + 2 * G * tm + T * k) + (512 * 80 if tm == 80 else 512 * 64) * 1024
+    got = L.mi_moe_prefill_workspace(*_pair(pkg, "IQ3_S", "IQ3_S", E, I, D), T, k, -1)
+    assert need <= got < need + (1 << 14)
