@@ -442,7 +442,8 @@ def route(x, router_w, bias, k, norm_topk=True, scaling=1.0, workspace=None):
     if router_w.shape[0] != D or (bias is not None and tuple(bias.shape) != (E,)):
         raise ValueError("route: router_w must be [D, E] = [%d, E] and bias [E]" % D)
     if workspace is None:
-        workspace = WORKSPACES.get("route", lib().mi_moe_route_workspace(N, D, E))
+        # the call's own: the second launch reads what the first left in it, and a captured call keeps its address
+        workspace = torch.empty(max(lib().mi_moe_route_workspace(N, D, E), 1), dtype=torch.uint8, device=x.device)
     idx = torch.empty((N, k), dtype=torch.int32, device=x.device)
     w = torch.empty((N, k), dtype=torch.float32, device=x.device)
     check("mi_moe_route", lib().mi_moe_route(_ptr(x), _ptr(router_w), _ptr(bias), N, D, E, int(k),
