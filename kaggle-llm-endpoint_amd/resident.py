@@ -634,7 +634,8 @@ def _mlp_many(x, ws3, scales, gu_form, down_form, D, I, limit, yb, yf, workspace
         if ws.numel() < need or ws.data_ptr() % 16:
             return False
     else:
-        ws = WORKSPACES.get("mlp_many", need)
+        # the call's own: a kept one would grow with B and leave a captured call with the address of a freed buffer
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device)
     for b0 in range(0, B, _MLP_MANY_STEP):
         n = min(_MLP_MANY_STEP, B - b0)
         check("mi_mlp_many", lib().mi_mlp_many(_ptr(_rows(x, b0, n)), n, D, I, _ptr(ws3[0]), _ptr(scales[0]), _ptr(ws3[1]),

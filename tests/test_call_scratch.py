@@ -57,3 +57,11 @@ def test_route(pkg, stand_in):
     fake = stand_in("mi_moe_route", 11)
     x, rw = torch.zeros((3, 64), dtype=torch.bfloat16), torch.zeros((64, 8))
     _own_scratch(fake, lambda: pkg.route(x, rw, None, 2))
+
+
+def test_many_token_mlp(pkg, stand_in):
+    fake = stand_in("mi_mlp_many", 15)
+    D, I = 256, 256
+    x = torch.zeros((33, D), dtype=torch.bfloat16)
+    leaves = [pkg.bf16_leaf(torch.zeros(s, dtype=torch.bfloat16), device="cpu") for s in ((D, I), (D, I), (I, D))]
+    _own_scratch(fake, lambda: pkg.bf16_mlp(x, *leaves, 7.0))

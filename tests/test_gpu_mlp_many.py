@@ -85,3 +85,32 @@ def test_mlp_many_last_piece(pkg, gpu):
         want = torch.cat([pkg.bf16_mlp(x[:4096], *leaves, 7.0), pkg.bf16_mlp(x[4096:], *leaves, 7.0)])
         torch.cuda.synchronize()
     assert torch.equal(got[0], want) and torch.equal(got[1], want)
+
+
+def test_mlp_many_and_route_captured(pkg, gpu):
+    """A captured MLP of 64 tokens and a captured router call, replayed between eager calls of more tokens on the capture
+    stream: every replay gives the eager bits."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(12)
+    D, I, E, k = 1024, 512, 64, 8
+    w = [torch.randn(s, device="cuda", generator=gen).to(torch.bfloat16) * 0.02 for s in ((D, I), (D, I), (I, D))]
+    leaves = [pkg.bf16_leaf(v) for v in w]
+    rw = torch.randn((D, E), device="cuda", generator=gen) / 32
+    x = torch.randn((64, D), device="cuda", generator=gen).to(torch.bfloat16)
+    more = torch.randn((700, D), device="cuda", generator=gen).to(torch.bfloat16)
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        want = (pkg.bf16_mlp(x, *leaves, 7.0), *pkg.route(x, rw, None, k))
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            got = (pkg.bf16_mlp(x, *leaves, 7.0), *pkg.route(x, rw, None, k))
+        for _ in range(4):
+            eager = pkg.bf16_mlp(more, *leaves, 7.0), pkg.route(more, rw, None, k)
+            for t in got:
+                t.zero_()
+            graph.replay()
+            stream.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
+            del eager
