@@ -665,8 +665,10 @@ def int8_mlp(x, gate, up, down, limit, want_f32=False, y_bf16=None, y_f32=None, 
     yb = y_bf16 if y_bf16 is not None else torch.empty((B, D), dtype=torch.bfloat16, device=x.device)
     yf = y_f32 if y_f32 is not None else (
         torch.empty((B, D), dtype=torch.float32, device=x.device) if want_f32 else None)
-    if _mlp_many(x, (g[0], u[0], d[0]), (g[1], u[1], d[1]), int(g[2]) | gt, int(d[2]) | dt, D, I, limit, yb, yf,
-                 workspace):
+    # other scale forms (mi_mlp_many's code of bf16 weights among them) are refused by the calls below, whatever B is
+    known = all(int(l[2]) & ~_lib.MI_I8_TILED in (_lib.MI_I8_ROW_SCALES, _lib.MI_I8_COL_SCALES) for l in (g, d))
+    if known and _mlp_many(x, (g[0], u[0], d[0]), (g[1], u[1], d[1]), int(g[2]) | gt, int(d[2]) | dt, D, I, limit, yb, yf,
+                           workspace):
         return (yb, yf) if want_f32 else yb
     for b0 in range(0, B, 32):
         n = min(32, B - b0)

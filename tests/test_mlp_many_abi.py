@@ -2,6 +2,9 @@
 takes and refuses."""
 import ctypes
 
+import pytest
+import torch
+
 
 def test_mlp_many_validation(pkg):
     L, lib = pkg._lib.lib(), pkg._lib
@@ -31,3 +34,13 @@ def test_mlp_many_workspace_serves_fewer_tokens(pkg):
     for D, I in ((6144, 2048), (4096, 1536), (3072, 1280), (2048, 768), (256, 256), (65536, 256)):
         sizes = [size(b, D, I) for b in range(1, 4097)]
         assert all(a <= b for a, b in zip(sizes, sizes[1:])), (D, I)
+
+
+@pytest.mark.parametrize("B", [8, 33, 5000])
+@pytest.mark.parametrize("gu,down", [(2, 2), (1, 2), (2, 1), (3, 3), (1, 3), (7, 1)])
+def test_int8_mlp_refuses_other_scale_forms(pkg, B, gu, down):
+    """Scale forms that an MLP does not take (the lm_head's, and the code that mi_mlp_many has for bf16 weights) are a
+    ValueError before any launch, for every token count."""
+    q, s = torch.zeros((256, 256), dtype=torch.int8), torch.ones(256)
+    with pytest.raises(ValueError):
+        pkg.int8_mlp(torch.zeros((B, 256), dtype=torch.bfloat16), (q, s, gu), (q, s, gu), (q, s, down), 7.0)
