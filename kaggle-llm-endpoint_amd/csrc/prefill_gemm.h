@@ -624,10 +624,10 @@ struct PfKq {
             m = d * ((float)sb - 32.0f);                              // exact
             a = -4.0f * m;
         } else {
-            // the scale group's four values as a byte table: v = 0..3 -> bf16(v * m + a)
+            // the scale group's four values as a byte table: v = 0..3 -> bf16(v * m + a), 0 * m too (d may be infinite)
             m = d * (float)(sb & 15u);
             a = -(f16_bits_to_f32(u[4] >> 16) * (float)(sb >> 4));
-            const uint32_t c01 = pf_bf16_pair(a, m + a), c23 = pf_bf16_pair(fmaf(2.0f, m, a), fmaf(3.0f, m, a));
+            const uint32_t c01 = pf_bf16_pair(fmaf(0.0f, m, a), m + a), c23 = pf_bf16_pair(fmaf(2.0f, m, a), fmaf(3.0f, m, a));
             const uint32_t lo = perm(c23, c01, 0x06040200u), hi = perm(c23, c01, 0x07050301u);
             const uint2 l0 = pf_lookup4(lo, lo, hi, hi, t0), l1 = pf_lookup4(lo, lo, hi, hi, t1);
             return __builtin_bit_cast(bf16x8, make_uint4(l0.x, l0.y, l1.x, l1.y));
