@@ -192,15 +192,23 @@ struct PfShared {
 //   kSplit                                      whether the launch's last round of tasks is split into K pieces
 
 // CB3: 160-column tiles of the code-tile layout; codebook slots per 640-column super tile (cb3_tiles.h).
+//
+// Split: the last round's tasks in K pieces.  The code for it costs registers that the CB3 loop does not have, and every
+// piece stores and reads 80 KB of sums, so it is a kernel of its own, taken for rows of kPfCb3SplitTiles super tiles
+// and more.  Whole / split, one launch, us (the plan's blocks from 16 to 1000 tokens): gate/up of K = 6144 (10 super tiles)
+// 40 tokens 167 / 150, 100 173 / 161, 512 329 / 320, 1000 577 / 583; K = 4096 (7) 64 tokens 61.7 / 62.9, 333 105 / 102, 512
+// 148 / 150; K = 3072 (5) 64 tokens 53.5 / 55.4; down of K = 2048 (4) 100 tokens 91 / 95, 512 178 / 173; K = 1536 (3) 512
+// tokens 75 / 81; K = 768 (2) 40 tokens 19.8 / 25.0.
+constexpr int kPfCb3SplitTiles = 8;
+
+template <bool Split>
 struct PfCb3 {
     struct Table {
         uint4 cbl[kPfWaves * 5 * 64];            // per-wavefront codebook slots (20 KB)
     };
     static constexpr bool kLdsOnlyBarrier = false;
     static constexpr int kCols = kCb3TileCols;
-    // the last round's tasks split into K pieces: 71 blocks of the benchmarked layer are 2.2 rounds of workgroups (512
-    // tokens, a few calls in a row 527 -> 466 us; sustained, where the card's power sets the pace, 538 -> 516)
-    static constexpr bool kSplit = true;
+    static constexpr bool kSplit = Split;
     static constexpr int kRtw = kPfRtw, kWaves = kPfWaves;
     static constexpr int kQOff = 4;
     using Wave = Cb3Wave;
@@ -1073,7 +1081,10 @@ int launch_prefill(int qtype, dim3 grid, hipStream_t s, const PfArgs &a) {
         case MI_QT_Q2_K: launch_prefill_block<MODE, FORM, PfKq<false>>(grid, s, a); break;
         case MI_QT_Q3_K: launch_prefill_block<MODE, FORM, PfKq<true>>(grid, s, a); break;
         case MI_QT_CB3:
-            hipLaunchKernelGGL((prefill_kernel<MODE, PfCb3, FORM, kPfTT>), grid, dim3(64 * kPfWaves), 0, s, a);
+            if (a.K >= 4 * kCb3TileCols * (kPfCb3SplitTiles - 1) + 1)
+                hipLaunchKernelGGL((prefill_kernel<MODE, PfCb3<true>, FORM, kPfTT>), grid, dim3(64 * kPfWaves), 0, s, a);
+            else
+                hipLaunchKernelGGL((prefill_kernel<MODE, PfCb3<false>, FORM, kPfTT>), grid, dim3(64 * kPfWaves), 0, s, a);
             break;
         default: return MI_ERR_QTYPE;
     }

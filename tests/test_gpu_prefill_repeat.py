@@ -6,14 +6,14 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("qtype,E", [("CB3", 270), ("IQ4_XS", 392)])
-def test_repeated_calls_equal(pkg, gpu, qtype, E):
+@pytest.mark.parametrize("qtype,E,D", [("CB3", 270, 5120), ("IQ4_XS", 392, 2048)])
+def test_repeated_calls_equal(pkg, gpu, qtype, E, D):
     """One block of one row per expert, so every block ties with every other in the launch order, over several of the
-    plan's wavefronts.  D 2048, I 256 gives the gate/up launch 2 (CB3) or 4 workgroups per block, 540 or 1568 tasks: a
-    last round of 28 or 32 tasks on 512 or 768 slots, whose 14 or 8 blocks are each summed in 4 pieces."""
+    plan's wavefronts.  I 256 gives the gate/up launch 2 (CB3) or 4 workgroups per block, 540 or 1568 tasks: a last round
+    of 28 or 32 tasks on 512 or 768 slots, whose 14 or 8 blocks are each summed in 4 pieces."""
     gen = torch.Generator(device="cuda")
     gen.manual_seed(31)
-    D, I = 2048, 256
+    I = 256
     table = {"CB3": pkg.random_cb3_table,
              "IQ4_XS": lambda *a: pkg.resident.random_iq4xs_table(*a, scale=2e-5)}[qtype]
     gate, up, down = (table(E, R, K, gen) for R, K in ((I, D), (I, D), (D, I)))
