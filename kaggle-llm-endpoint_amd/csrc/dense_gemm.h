@@ -1,6 +1,6 @@
 // Dense GEMM of many tokens against int8 or bf16 weights on the gfx950 matrix cores: the gate/up and down products of
-// mlp_partial (model.py:125-127) and x @ W for more tokens than the streaming kernels of int8_project.hip take at once
-// (32).  Those read every weight once per 32 tokens; here a workgroup's weight tile is converted once and meets 64 or
+// mlp_partial (model.py:125-127) for more tokens than the streaming kernels of int8_project.hip take at once (32; the
+// single projections take them 32 at a time).  Those read every weight once per 32 tokens; here a workgroup's weight tile is converted once and meets 64 or
 // 128 tokens.
 //
 // Tile: 128 weight rows (PAIR: 64 of gate and the same 64 of up) x 32 NT tokens x 64 columns, 4 wavefronts as 2 x 2,

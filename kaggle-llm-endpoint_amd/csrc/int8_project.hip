@@ -477,6 +477,7 @@ static int i8_block_cols(int form) { return form == kW16 ? 64 : 128; }
 // 12 (3) 15.4; bf16 2048 -> 6144 1 token S = 2 (0.75) 10.3, 8 (3) 9.5, 8 tokens 9.9 and 10.7; bf16 3072 -> 2560 1 token S = 4
 // (0.63) 8.5, 6 (0.94) 7.4, 12 8.4.
 // More row groups: about 3 wavefronts per SIMD (3072 over 256 CUs) in flight.
+// The plans count on the whole chip's 256 CUs: on fewer they cost time, not results.
 //
 // Writes S[b - b0] for every token count b of b0 .. b1 (up to 32 of them).
 static void i8_splits_of(int b0, int b1, int n_in, int tiles, int scale_axis, int *S) {
@@ -676,7 +677,7 @@ static int mlp_launches(const uint16_t *x_bf16, int32_t B, int32_t D, int32_t I,
 // Tiles of 128 tokens reuse a converted weight twice as often as tiles of 64, but halve the workgroups: they pay from
 // about 24 steps of a 128 x 128 tile per CU on (D 6144, I 2048: 512 tokens 76 us against 82, 128 tokens 42 against 39;
 // D 2048, I 768 at 1500 tokens 48 against 45).
-// Splits fill the chip's two workgroups per CU, but every split writes and reads back f32 partials of the whole
+// Splits fill two workgroups on each of 256 CUs, but every split writes and reads back f32 partials of the whole
 // output: up to 192 workgroups a split pays down to 8 steps each (down, 64 tokens: 32 us with 4 splits, 36 with 2),
 // beyond that only with 24 steps left (gate/up at 512 tokens: 4 splits 76 us, 2 splits 81; down at 512 tokens, 32 steps
 // in all: 1 split 76, 2 splits 79).

@@ -181,14 +181,18 @@ struct PfShared {
 // D 6144, I 2048, 64 experts, top-8, same bits: IQ2_S + IQ4_XS 27 tokens 453 -> 330 us, 512 tokens 705 -> 577, IQ3_S
 // 1999 tokens 2288 -> 1919.
 //
-// A provider streams the weights of one wavefront's 64 rows (4 row tiles) of expert e, one column tile at a time, and
+// A provider streams the weights of one wavefront's kRtw row tiles of expert e, one column tile at a time, and
 // runs the tile's k-steps on the matrix cores against the staged activations.  Its state is two values the workgroup
 // body keeps as locals: Wave (addressing, fixed per wavefront) and Regs (the loads in flight).
 //   init(w, s, a, sh, mat, e, rg, wave, lane, st0, st1)   set up w for super tiles [st0, st1) (column tiles
 //                                               [4 st0, 4 st1)), issue the first column tiles' loads into s
 //   n_tiles(a, mat)                             column tiles of a row
-//   tile<NTT, C>(w, s, st, xt, acc)             column tile 4 st + C; xt = the staged tile at row jt, lane group q
-//   kCols, kQOff                                columns per tile; dwords between lane groups' activations in a step
+//   tile<NTT, C>(w, s, st, xt, acc)             column tile 4 st + C; xt = the staged tile at row jt, lane group q (CB3)
+//   tile<NTT, C>(w, s, st, xb, xoff, acc)       the same of the block formats; xb = the staged tile, xoff = the lane's byte
+//                                               offset of chunk act_chunk(q) of row jt
+//   kCols                                       columns per tile
+//   kRtw, kWaves                                row tiles per wavefront, wavefronts per workgroup
+//   kQOff (CB3)                                 dwords between lane groups' activations in a step
 //   kSplit                                      whether the launch's last round of tasks is split into K pieces
 
 // CB3: 160-column tiles of the code-tile layout; codebook slots per 640-column super tile (cb3_tiles.h).
@@ -901,7 +905,7 @@ __device__ __forceinline__ void prefill_body(const PfArgs &a, PfShared<WP, TT> &
         }
     }
 
-    // epilogue: lane (jt, q) holds rows 16 r + 4 q + i (i = 0..3) of the wavefront's 64 rows for tokens 16 t + jt
+    // epilogue: lane (jt, q) holds rows 16 r + 4 q + i (i = 0..3) of the wavefront's 16 kRtw rows for tokens 16 t + jt
     const int rbase = rg * 16 * kRtw;
     if constexpr (MODE == 0) {
         // gate accumulators of as many (gate, up) pairs as the activation buffers hold at once: [rows][kGPitch]

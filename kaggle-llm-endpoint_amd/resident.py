@@ -650,8 +650,10 @@ def int8_mlp(x, gate, up, down, limit, want_f32=False, y_bf16=None, y_f32=None, 
     """mlp_partial over int8 leaves (model.py:125-127 with quant8.py:91-99): y = bf16(h @ Wd) with
     h = bf16(swiglu_clamped(bf16(x @ Wg), bf16(x @ Wu))), W = bf16(f32(q) * s).  x bf16 [B, D]; gate, up, down:
     reference leaves {"q", "s"} or int8_leaf triples (qT, s, scale_axis); gate and up share one scale form.
-    -> y bf16 [B, D] (and y f32, the down projection before its rounding, with want_f32).  Tokens go 32 per call
-    (mi_int8_mlp's limit); preallocated outputs / workspace make each call allocation-free.
+    -> y bf16 [B, D] (and y f32, the down projection before its rounding, with want_f32).  Up to 32 tokens are one call
+    of mi_int8_mlp.  More go to mi_mlp_many (4096 a call), or 32 at a time where a pointer is off its alignment or a kept
+    ``workspace`` is too small for it (256 KB + mi_mlp_many_workspace).  Preallocated outputs and a workspace that fits
+    make the call allocation-free.
     The workspace's first 256 KB are completion counters that must be zero before its first int8 call (a
     zero-filled allocation; every call leaves them zero again): a workspace left nonzero gives wrong sums, silently."""
     g, u, d = [int8_leaf(l, x.device) if isinstance(l, dict) else l for l in (gate, up, down)]
@@ -731,8 +733,9 @@ def bf16_project(x, w, want_f32=False, y_bf16=None, y_f32=None, workspace=None):
 def bf16_mlp(x, gate, up, down, limit, want_f32=False, y_bf16=None, y_f32=None, workspace=None):
     """mlp_partial over bf16 leaves (model.py:125-127): y = bf16(h @ Wd) with h = bf16(swiglu_clamped(bf16(x @ Wg),
     bf16(x @ Wu))).  x bf16 [B, D]; gate, up: W bf16 [D, I], down: W bf16 [I, D] (reference leaves) or Bf16Leaf.
-    -> y bf16 [B, D] (and y f32, the down projection before its rounding, with want_f32).  Tokens go 32 per call
-    (mi_bf16_mlp's limit); preallocated outputs / workspace make each call allocation-free.
+    -> y bf16 [B, D] (and y f32, the down projection before its rounding, with want_f32).  Up to 32 tokens are one call
+    of mi_bf16_mlp; more go the way of int8_mlp.  Preallocated outputs and a workspace that fits make the call
+    allocation-free.
     The workspace's first 256 KB are completion counters that must be zero before its first call (a zero-filled
     allocation; every call leaves them zero again)."""
     g, u, d = [bf16_leaf(l, x.device).wT for l in (gate, up, down)]
