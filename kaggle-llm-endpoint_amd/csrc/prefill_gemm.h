@@ -177,7 +177,7 @@ struct PfShared {
 // tiles per decoded weight they, not the MFMAs, set the pace.  Per 8 weights (a lane's A operand) the loops issue
 // (vector instructions / table gathers, before -> now): IQ2_S 44 / 2 x 16 bytes -> 25 / 8 bytes (levels through a
 // byte-permute table of the three scaled levels and their negatives), IQ3_S 41 / 3 x 16 -> 31 / 2 x 8, IQ4_XS 35 /
-// 4 x 8 -> 23 / 4 x 4 (f16 levels widened inside the multiply), Q2_K 48 -> 27 (byte-permute table).  Measured at
+// 4 x 8 -> 23 / 4 x 4 (f16 levels widened inside the multiply), Q2_K 48 -> 28 (byte-permute table).  Measured at
 // D 6144, I 2048, 64 experts, top-8, same bits: IQ2_S + IQ4_XS 27 tokens 453 -> 330 us, 512 tokens 705 -> 577, IQ3_S
 // 1999 tokens 2288 -> 1919.
 //
